@@ -2017,10 +2017,10 @@ __global__ __launch_bounds__(256) void k_den_finish(BuildArgs a, const DenFinish
 // through s_t (2 x 64 x 64 doubles, the chunk buffers, free after the first
 // barrier): wavefront 1 (the lower-left quadrant) hands its entries to
 // wavefront 2 (upper-right), and the two diagonal quadrants (wavefronts 0 and
-// 3) each transpose their own.  The fold pays where the atomics are exposed
-// (k_vxc_gemm_f32: 2.5 ms of 23.8 on (H2O)128 / def2-SVP); in the
-// register-staged kernels they drain behind other workgroups' staging and
-// the fold's barriers cost more than it saves.
+// 3) each transpose their own.  The fold pays in the directly loaded kernels
+// (k_vxc_gemm_f32: 2.5 ms of 23.8 on (H2O)128 / def2-SVP; k_vxc_dma: 0.3 ms of
+// 3.6 on (H2O)32); in the register-staged ones the atomics drain behind other
+// workgroups' staging and the fold's barriers cost more than it saves.
 template <bool F32, bool FOLD>
 __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem &it,
                                             const LeafDev &L, const MolDev &MD,
@@ -2068,8 +2068,14 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
     const int nu = it.c0 + wcw * hc + 16 * j + l16;
     co[j] = j < CT && nu < L.m ? map[nu] : -1;
   }
+  // FP64: the two terms of a folded entry are screened one by one, as the
+  // unfolded scatter screens them, so the fold drops nothing more
+  auto kept = [&](double v) __attribute__((always_inline)) {
+    return F32 || fabs(v) >= cut ? v : 0.0;
+  };
   auto emit = [&](int i, int j, int r, double v) __attribute__((always_inline)) {
-    if (ro[i][r] >= 0 && co[j] >= 0 && fabs(v) >= cut) atomicAdd(Km + ro[i][r] + co[j], v);
+    if (ro[i][r] >= 0 && co[j] >= 0 && (F32 ? fabs(v) >= cut : v != 0.0))
+      atomicAdd(Km + ro[i][r] + co[j], v);
   };
   // [row][col ^ (row % 16)] keeps a wavefront's column reads off one bank
   auto tix = [](int row, int col) { return row * 64 + (col ^ (row & 15)); };
@@ -2096,8 +2102,8 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int lr = lrow(i, r), lc = 16 * j + l16;
-          if (lr < lc) emit(i, j, r, acc[i][j][r] + T[tix(lc, lr)]);
-          else if (lr == lc) emit(i, j, r, acc[i][j][r]);
+          if (lr < lc) emit(i, j, r, kept(acc[i][j][r]) + kept(T[tix(lc, lr)]));
+          else if (lr == lc) emit(i, j, r, kept(acc[i][j][r]));
         }
       }
     }
@@ -2119,7 +2125,8 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
       for (int j = 0; j < 4; ++j) {
         if (j >= CT) break;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) emit(i, j, r, acc[i][j][r] + R0[tix(16 * j + l16, lrow(i, r))]);
+        for (int r = 0; r < 4; ++r)
+          emit(i, j, r, kept(acc[i][j][r]) + kept(R0[tix(16 * j + l16, lrow(i, r))]));
       }
     }
   }
@@ -2129,31 +2136,25 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
   }
 }
 
-// Vxc item, block pair (r, c) of a leaf: the leaf's points are streamed kTVp
-// at a time; each chunk stages Phi and A = c0 Phi + c . grad Phi
-// (xc_potential_matrix.cpp:19-41) of the block rows in LDS ([row][point]),
-// and wavefront (wr, wc) accumulates its quadrant of
+// dS item (FP32 storage, context set-up), block pair (r, c) of a leaf: the
+// leaf's points are streamed kTVp at a time; each chunk stages Phi and A = w r
+// (r the value plane's rounding residuals) of the block rows in LDS
+// ([row][point]), and wavefront (wr, wc) accumulates its quadrant of
 //   r == c:  K_rr = Phi_r^T A_r
 //   r <  c:  V_rc = Phi_r^T A_c + A_r^T Phi_c
 // in registers.  Entry (mu, nu) is added to K(map[nu], map[mu]) with FP64
-// atomics; Vxc = K + K^T afterwards counts every entry of V_loc once.
-// RES (FP32 storage, context set-up): A = w r with r the value plane's
-// rounding residuals, so K + K^T = dS = sum_p w_p (r Phi^T + Phi r^T); only
-// the items of the leaves [res_leaf0, res_leaf1) whose residuals a.ao_res
-// holds run, and entries below kStorageCut are not added.
-template <typename S, bool GGA, bool RES = false>
-__global__ __launch_bounds__(256, 2) void k_vxc_tile(BuildArgs a, const S *__restrict__ ao,
-                                                     const VxcItem *__restrict__ items) {
-  // the four operand buffers in one array: the scatter's transposes reuse it
+// atomics, so K + K^T = dS = sum_p w_p (r Phi^T + Phi r^T).  Only the items of
+// the leaves [res_leaf0, res_leaf1) whose residuals a.ao_res holds run, and
+// entries below kStorageCut are not added.
+__global__ __launch_bounds__(256, 2) void k_vxc_overlap(BuildArgs a, const float *__restrict__ ao,
+                                                        const VxcItem *__restrict__ items) {
   __shared__ __align__(16) double s_stage[4 * kTileAo * kTVld];
-  static_assert(4 * kTileAo * kTVld >= 2 * 64 * 64, "scatter transposes fit");
   // buffer offsets: Phi rows 0, A rows kB, Phi columns 2 kB, A columns 3 kB
   constexpr int kB = kTileAo * kTVld;
-  __shared__ double s_c[2][4][kTVp];
+  __shared__ double s_w[2][kTVp];
   const VxcItem it = items[blockIdx.x];
   if (it.leaf < 0 || !a.leaf_active[it.leaf]) return;
-  if constexpr (RES)
-    if (it.leaf < a.res_leaf0 || it.leaf >= a.res_leaf1) return;
+  if (it.leaf < a.res_leaf0 || it.leaf >= a.res_leaf1) return;
   const LeafDev L = a.leaves[it.leaf];
   const MolDev MD = a.mols[L.mol];
   double *Km = a.K + MD.moff;
@@ -2164,18 +2165,16 @@ __global__ __launch_bounds__(256, 2) void k_vxc_tile(BuildArgs a, const S *__res
   const bool diag = it.r0 == it.c0;
   const int hr = it.wr >> 1, hc = it.wc >> 1;
   const int RT = hr >> 4, CT = hc >> 4;
-  const S *phi = ao + L.ao_off;
-  const long long cs = (long long)L.mp * L.np;
+  const float *phi = ao + L.ao_off;
+  const float *res = a.ao_res + (L.res_off - a.res_base);
   const int nrow = diag ? it.wr : it.wr + it.wc;
-  static_assert(!RES || (!GGA && std::is_same<S, float>::value), "dS: FP32 storage, LDA form");
-  const double *cf = RES ? a.pw + L.pt_off : a.coef + L.pt_off;
-  constexpr int NQ = GGA ? 4 : 1;
+  const double *wt = a.pw + L.pt_off;
   d4 acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-  if (t < NQ * kTVp) s_c[0][t / kTVp][t % kTVp] = cf[(t / kTVp) * a.ptot + t % kTVp];
+  if (t < kTVp) s_w[0][t] = wt[t];
   const int xo = (wr * hr + l16) * kTVld + 4 * g, yo = (wcw * hc + l16) * kTVld + 4 * g;
   // one point loop per tile shape
   tile_shape(RT, CT, [&](auto R, auto C) __attribute__((always_inline)) {
@@ -2184,32 +2183,17 @@ __global__ __launch_bounds__(256, 2) void k_vxc_tile(BuildArgs a, const S *__res
   // padding points
   for (int p0 = 0; p0 < L.n; p0 += kTVp, buf ^= 1) {
     __syncthreads();
-    // the next chunk's coefficients (read after the barrier below)
-    if (p0 + kTVp < L.n && t < NQ * kTVp)
-      s_c[buf ^ 1][t / kTVp][t % kTVp] = cf[(t / kTVp) * a.ptot + p0 + kTVp + t % kTVp];
+    // the next chunk's weights (read after the barrier below)
+    if (p0 + kTVp < L.n && t < kTVp) s_w[buf ^ 1][t] = wt[p0 + kTVp + t];
     for (int gi = t; gi < nrow * (kTVp / 4); gi += 256) {
       const int row = gi >> 2, p = 4 * (gi & 3);
       const bool rb = row < it.wr;
       const int mu = rb ? it.r0 + row : it.c0 + row - it.wr;
       const long long o = (long long)mu * L.np + p0 + p;
-      const d4 f = load4_as<double>(phi + o);
+      const d4 f = load4_as<double>(phi + o), r = load4_as<double>(res + o);
       d4 A;
-      if constexpr (RES) {
-        const d4 r = load4_as<double>(a.ao_res + (L.res_off - a.res_base) + o);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) A[e] = s_c[buf][0][p + e] * r[e];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) A[e] = s_c[buf][0][p + e] * f[e];
-      }
-      if constexpr (GGA) {
-        const d4 fx = load4_as<double>(phi + cs + o);
-        const d4 fy = load4_as<double>(phi + 2 * cs + o);
-        const d4 fz = load4_as<double>(phi + 3 * cs + o);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          A[e] += s_c[buf][1][p + e] * fx[e] + s_c[buf][2][p + e] * fy[e] + s_c[buf][3][p + e] * fz[e];
-      }
+      for (int e = 0; e < 4; ++e) A[e] = s_w[buf][p + e] * r[e];
       const int lr = rb ? row : row - it.wr;
       *reinterpret_cast<d4u *>(s_stage + (rb ? 0 : 2 * kB) + lr * kTVld + p) = f;
       *reinterpret_cast<d4u *>(s_stage + (rb ? kB : 3 * kB) + lr * kTVld + p) = A;
@@ -2227,7 +2211,7 @@ __global__ __launch_bounds__(256, 2) void k_vxc_tile(BuildArgs a, const S *__res
     if (!diag) product(kB, 2 * kB);
   }
   });
-  vxc_scatter<false, false>(acc, it, L, MD, map, Km, RES ? kStorageCut : kScatterCut, s_stage);
+  vxc_scatter<false, false>(acc, it, L, MD, map, Km, kStorageCut, s_stage);
 }
 
 // FP32 form of the Vxc item (FP32 mode): the same block pairs with Phi and
@@ -2492,6 +2476,220 @@ __global__ __launch_bounds__(256, 2) void k_vxc_gemm_f32(BuildArgs a, const floa
   vxc_scatter<true, true>(acc, it, L, MD, map, Km, kScatterCut, reinterpret_cast<double *>(s_stage));
 }
 
+// Workgroup barrier for LDS hand-offs only: waits for this wavefront's LDS
+// accesses (lgkmcnt) but not for its outstanding global memory operations,
+// so the MFMA wavefronts' scatter atomics drain while the next steps run
+// (__syncthreads would wait for them at every step).  The empty asm
+// statements keep the compiler from moving memory accesses across it.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // vmcnt and expcnt: no wait; lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+// Vxc item in FP64 (FP64 / FP32-cache contexts), block pair (r, c) of a leaf,
+// the raw AO planes staged by direct-to-LDS loads.  A chunk is 64 bytes of
+// every staged AO row and plane: vd_pts() points (8 with FP64 storage, 16 with
+// FP32), rows as in k_vxc_gemm_f32 (16-byte slot of point group q in row R at
+// q ^ ((R / 2) % 4)).  Wavefront (wr, wc) reads its operands of 8 points (two
+// k-steps) and forms A = c0 Phi + c . grad Phi (xc_potential_matrix.cpp:19-41)
+// of its rows and columns in registers:
+//   r == c:  K_rr = Phi_r^T A_r
+//   r <  c:  V_rc = Phi_r^T A_c + A_r^T Phi_c   (LDA: Phi_r^T (2 c0 Phi_c))
+// TAU adds the meta-GGA's sum_k d_k Phi_r^T (c_tau d_k Phi_c)
+// (xc_potential_matrix.cpp:44-58), c_tau doubled for r < c (V = K + K^T counts
+// an off-diagonal item once), from the planes already staged: five products
+// per chunk for one set of loads.
+// After a chunk's last operand read the buffer is released (barrier) and the
+// next chunk's loads are issued, so they run under this chunk's MFMAs: one
+// buffer of 64 KB suffices and two workgroups share a CU (up to four smaller
+// buffers in flight, where the item's rows allow them, measured 2 % slower).
+// Bound by the FP64 MFMAs and by HBM together: on (H2O)32 / def2-SVP / PBE
+// 3.25 ms for 9.45e10 flops and 1.2e10 bytes fetched and written (matrix cores
+// busy 37 %, 3.7 TB/s).  Forming Phi and A in LDS by way of registers (each
+// element's four planes loaded and waited for by the thread that stores it)
+// took 4.12 ms there; the meta-GGA's passes of per-leaf kernels 23.7 ms, this
+// form 6.46 ms (2.9 times the MFMAs; its scatter drops nothing above 1e-18).  A chunk's operands fill the registers (128 of the 256
+// hold accumulators): Phi is read last, and TAU keeps its plane loop rolled,
+// without which 18 and 40 of them spill.
+constexpr int kVdRow = 64;                         // bytes of a row in a chunk
+constexpr int kVdPlane = 2 * kTileAo * kVdRow;     // bytes of one plane's rows
+template <typename S> constexpr int vd_pts() { return kVdRow / (int)sizeof(S); }
+// coefficients of a chunk behind the planes: [planes][points] doubles
+template <typename S, bool GGA, bool TAU> constexpr int vd_smem() {
+  return (GGA ? 4 : 1) * kVdPlane + (GGA ? 4 + (TAU ? 1 : 0) : 1) * vd_pts<S>() * 8;
+}
+
+template <typename S, bool GGA, bool TAU>
+__device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__restrict__ ao,
+                                             const int *__restrict__ ao_map, const VxcItem &it,
+                                             char *s_stage) {
+  static_assert(GGA || !TAU, "tau terms come with the GGA planes");
+  constexpr int PT = vd_pts<S>(), NQ = GGA ? 4 : 1, NC = NQ + (TAU ? 1 : 0);
+  constexpr int NH = PT / 8;  // operand rounds of 8 points per chunk
+  const LeafDev L = a.leaves[it.leaf];
+  const MolDev MD = a.mols[L.mol];
+  double *Km = a.K + MD.moff;
+  const int *map = ao_map + L.map_off;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int wr = wave & 1, wcw = wave >> 1;
+  const bool diag = it.r0 == it.c0;
+  const int hr = it.wr >> 1, hc = it.wc >> 1;
+  const S *phi = ao + L.ao_off;
+  const long long cs = (long long)L.mp * L.np;
+  // 16-row groups of the row block, then of the column block, that hold real
+  // AOs; the columns' rows start at LDS row cb (0 for a diagonal item)
+  const int cb = diag ? 0 : it.wr;
+  const int gr = (min((int)it.wr, L.m - it.r0) + 15) >> 4;
+  const int gc = diag ? 0 : (min((int)it.wc, L.m - it.c0) + 15) >> 4;
+  // loads: lane l takes row l / 4 of a group, slot l % 4 (16 bytes)
+  const int lrow = lane >> 2;
+  const long long loff = (long long)lrow * L.np + (16 / (int)sizeof(S)) * ((lane & 3) ^ vxc_swz(lrow));
+  const double *cptr = nullptr;  // wavefront 0's coefficient lanes
+  if (wave == 0 && lane < NC * (PT / 2)) {
+    const int q = lane / (PT / 2);
+    cptr = (TAU && q == NQ ? a.coef_tau : a.coef + q * a.ptot) + L.pt_off + 2 * (lane % (PT / 2));
+  }
+  auto dma = [&](int p0) __attribute__((always_inline)) {
+    const int q0 = GGA ? wave : 0;
+    const S *src = phi + q0 * cs + loff + p0;
+    char *dst = s_stage + q0 * kVdPlane;
+    for (int k = GGA ? 0 : wave; k < gr + gc; k += GGA ? 1 : 4) {
+      const int lr = k < gr ? 16 * k : cb + 16 * (k - gr);
+      const int ar = k < gr ? it.r0 + 16 * k : it.c0 + 16 * (k - gr);
+      __builtin_amdgcn_global_load_lds(src + (long long)ar * L.np, dst + lr * kVdRow, 16, 0, 0);
+    }
+    if (wave == 0 && lane < NC * (PT / 2))
+      __builtin_amdgcn_global_load_lds(cptr + p0, s_stage + NQ * kVdPlane, 16, 0, 0);
+  };
+  const int nch = (L.n + PT - 1) / PT;
+  const int RTl = live_tiles(L.m - (it.r0 + wr * hr), hr), CTl = live_tiles(L.m - (it.c0 + wcw * hc), hc);
+  if (nch > 0) dma(0);
+  d4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+  // this lane's operand bytes of row tile 0 / column tile 0 in plane 0
+  const char *xr = s_stage + (wr * hr + l16) * kVdRow + ((g ^ vxc_swz(l16)) << 4);
+  const char *xc = s_stage + (cb + wcw * hc + l16) * kVdRow + ((g ^ vxc_swz(l16)) << 4);
+  const double *sc = reinterpret_cast<const double *>(s_stage + NQ * kVdPlane) + (PT / 4) * g;
+  auto ld = [](const char *p, int h) __attribute__((always_inline)) -> d2u {
+    if constexpr (sizeof(S) == 8) {
+      return *reinterpret_cast<const d2u *>(p);
+    } else {
+      typedef float f2 __attribute__((ext_vector_type(2)));
+      const f2 v = *reinterpret_cast<const f2 *>(p + 8 * h);
+      return d2u{(double)v[0], (double)v[1]};
+    }
+  };
+  tile_shape_ext(RTl, CTl, [&](auto R, auto C) __attribute__((always_inline)) {
+    constexpr int NR = decltype(R)::value, NCt = decltype(C)::value;
+    constexpr int NRs = NR ? NR : 1, NCs = NCt ? NCt : 1;
+    for (int c = 0; c < nch; ++c) {
+      vmcnt_barrier<0>();  // the chunk is staged
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        // A of the columns (Phi_r^T A_c), and of the rows for the transpose
+        // term; Phi last, so that fewer operands are held at once
+        d2u pr[NRs], ar[NRs], pc[NCs], ac[NCs];
+        auto coef = [&](int q) __attribute__((always_inline)) {
+          return *reinterpret_cast<const d2u *>(sc + q * PT + 2 * h);
+        };
+        if constexpr (GGA) {
+          d2u ct{};
+          if constexpr (TAU) {
+            ct = coef(NQ);
+            if (!diag) ct = ct + ct;
+          }
+#pragma unroll
+          for (int j = 0; j < NCt; ++j) ac[j] = d2u{0.0, 0.0};
+#pragma unroll
+          for (int i = 0; i < NR; ++i) ar[i] = d2u{0.0, 0.0};
+          // the tau form's products per plane fill the pipeline; unrolled, the
+          // planes' operands spill
+#pragma unroll TAU ? 1 : 3
+          for (int k = 1; k < 4; ++k) {
+            const d2u ck = coef(k);
+            d2u xk[NRs], yk[NCs];
+#pragma unroll
+            for (int j = 0; j < NCt; ++j) {
+              yk[j] = ld(xc + k * kVdPlane + 16 * j * kVdRow, h);
+              ac[j] += ck * yk[j];
+            }
+            if (TAU || !diag) {
+#pragma unroll
+              for (int i = 0; i < NR; ++i) {
+                xk[i] = ld(xr + k * kVdPlane + 16 * i * kVdRow, h);
+                ar[i] += ck * xk[i];
+              }
+            }
+            if constexpr (TAU) {
+#pragma unroll
+              for (int j = 0; j < NCt; ++j) yk[j] = ct * yk[j];
+#pragma unroll
+              for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int i = 0; i < NR; ++i)
+#pragma unroll
+                  for (int j = 0; j < NCt; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(xk[i][s], yk[j][s], acc[i][j], 0, 0, 0);
+            }
+          }
+        }
+        d2u c0 = coef(0);
+        if (!GGA && !diag) c0 = c0 + c0;
+#pragma unroll
+        for (int j = 0; j < NCt; ++j) {
+          pc[j] = ld(xc + 16 * j * kVdRow, h);
+          if constexpr (GGA) ac[j] += c0 * pc[j];
+          else ac[j] = c0 * pc[j];
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+          pr[i] = ld(xr + 16 * i * kVdRow, h);
+          if (GGA && !diag) ar[i] += c0 * pr[i];
+        }
+        if (h == NH - 1 && c + 1 < nch) {
+          lds_barrier();  // every wavefront holds its operands: the buffer is free
+          dma((c + 1) * PT);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int i = 0; i < NR; ++i)
+#pragma unroll
+            for (int j = 0; j < NCt; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[i][s], ac[j][s], acc[i][j], 0, 0, 0);
+        if constexpr (GGA) {
+          if (!diag) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+              for (int i = 0; i < NR; ++i)
+#pragma unroll
+                for (int j = 0; j < NCt; ++j)
+                  acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[i][s], pc[j][s], acc[i][j], 0, 0, 0);
+          }
+        }
+      }
+    }
+  });
+  vxc_scatter<false, GGA>(acc, it, L, MD, map, Km, TAU ? kStorageCut : kScatterCut, reinterpret_cast<double*>(s_stage));
+}
+
+template <typename S, bool GGA, bool TAU>
+__global__ __launch_bounds__(256, 2) void k_vxc_dma(BuildArgs a, const S *__restrict__ ao,
+                                                    const int *__restrict__ ao_map,
+                                                    const VxcItem *__restrict__ items) {
+  __shared__ __align__(16) char s_stage[vd_smem<S, GGA, TAU>()];
+  const VxcItem it = items[blockIdx.x];
+  if (it.leaf < 0 || !a.leaf_active[it.leaf]) return;
+  vxc_item_dma<S, GGA, TAU>(a, ao, ao_map, it, s_stage);
+}
+
 // Persistent, wavefront-specialised form of the Vxc items: one 512-thread
 // workgroup per CU walks the items blockIdx.x, blockIdx.x + gridDim.x, ...
 // (the same XCD for all of them, gridDim.x being a multiple of 8) chunk by
@@ -2530,17 +2728,6 @@ __device__ __forceinline__ void vxc_next(const BuildArgs &a, const VxcItem *item
 
 constexpr int kWsBuf = 4 * kTileAo * kTVld;  // doubles per staging buffer
 
-// Workgroup barrier for LDS hand-offs only: waits for this wavefront's LDS
-// accesses (lgkmcnt) but not for its outstanding global memory operations,
-// so the MFMA wavefronts' scatter atomics drain while the next steps run
-// (__syncthreads would wait for them at every step).  The empty asm
-// statements keep the compiler from moving memory accesses across it.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // vmcnt and expcnt: no wait; lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 static size_t vxc_ws_smem() { return sizeof(double) * 2 * kWsBuf; }
 
 template <typename S, bool GGA>
@@ -3058,9 +3245,9 @@ void run_storage_overlap(const ContractPlan &plan, const BuildArgs &a, const voi
   if (plan.vxc_items.get() == nullptr || a.ao_res == nullptr)
     throw Error(OCCXC_ERR_INTERNAL, "storage overlap: needs the Vxc item list and the residuals");
   if (plan.n_vxc_items == 0) return;
-  k_vxc_tile<float, false, true><<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const float *>(ao),
-                                                                  plan.vxc_items.get());
-  check_launch("k_vxc_tile (dS)");
+  k_vxc_overlap<<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const float *>(ao),
+                                                 plan.vxc_items.get());
+  check_launch("k_vxc_overlap");
 }
 
 void run_vxc_reduce(const BuildArgs &a, double *V, hipStream_t s) {
@@ -3104,9 +3291,10 @@ void run_vxc(const ContractPlan &plan, const BuildArgs &a, const void *ao, int p
         check_launch("k_vxc_ws");
         return;
       }
-      (a.deriv ? k_vxc_tile<S, true> : k_vxc_tile<S, false>)
-          <<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const S *>(ao), plan.vxc_items.get());
-      check_launch("k_vxc_tile");
+      (a.deriv ? k_vxc_dma<S, true, false> : k_vxc_dma<S, false, false>)
+          <<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const S *>(ao), a.ao_map,
+                                            plan.vxc_items.get());
+      check_launch("k_vxc_dma");
     };
     if (precision == 0) launch(double{});
     else launch(float{});
@@ -3152,6 +3340,17 @@ void run_vxc_mgga(const ContractPlan &plan, const BuildArgs &a, const LeafDev *l
   check_coef_planes(4, a.coef_planes, "meta-GGA Vxc stage (GGA term)");
   check_coef_planes(1, a.coef_tau_planes, "meta-GGA Vxc stage (tau terms)");
   if (a.nleaves == 0) return;
+  if (plan.tiled) {
+    // the GGA term and the three tau terms of a block pair in one item
+    if (precision == 0)
+      k_vxc_dma<double, true, true><<<plan.n_vxc_items, 256, 0, s>>>(
+          a, static_cast<const double *>(ao), a.ao_map, plan.vxc_items.get());
+    else
+      k_vxc_dma<float, true, true><<<plan.n_vxc_items, 256, 0, s>>>(
+          a, static_cast<const float *>(ao), a.ao_map, plan.vxc_items.get());
+    check_launch("k_vxc_dma (meta-GGA)");
+    return;
+  }
   // leaves of up to kSymMaxMp AOs: the GGA term and the three tau terms in
   // one symmetric launch; the others: the general kernel on the GGA term and
   // on each derivative plane (LDA form, tau coefficients)

@@ -1,0 +1,79 @@
+"""The tiled contractions at the edges of their tiles: leaves of fewer points
+than a chunk or a block, AO counts around the 16- and 32-row tile steps, one
+to four blocks per leaf, every form (LDA, GGA, meta-GGA; one spin and two)
+and both storage precisions, against the CPU oracle.
+
+Bounds on Vxc in FP64: each leaf drops at most two terms below 1e-14 per
+entry (none above 1e-18 for a meta-GGA) and the sums round at 1e-15 of the
+largest entry per leaf, so 2e-14 leaves + 1e-13 max|V|, below 1e-11 here.
+FP32 AO storage rounds each value by 6e-8 relative: 1e-7 max|V|, the bound of
+the batch tests."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import random_density
+from occ_amd import AOBasis, molecules
+from occ_amd.dft import XCContext, functional_ids
+from occ_amd.grid import GridSettings, MolecularGrid
+
+pytestmark = pytest.mark.gpu
+
+SYSTEMS = {"water": lambda: molecules.water(), "methane": lambda: molecules.alkane(1),
+           "water3": lambda: molecules.water_cluster(3, seed=6),
+           "alkane5": lambda: molecules.alkane(5)}
+
+
+def _setup(system, basis_name, method, precision, tile, nrad=19, nang=38):
+    atoms = SYSTEMS[system]()
+    basis = AOBasis.load(atoms, basis_name, pure=basis_name.startswith("def2"))
+    pts, wts = MolecularGrid(atoms, GridSettings(radial_points=nrad, angular_points=nang)).build()
+    print(f"{system} {basis_name} {method} {precision} tile {tile}: nbf={basis.nbf} "
+          f"npts={len(wts)}", flush=True)
+    ctx = XCContext(basis, pts, wts, functional_ids(method), precision=precision, tile_ao=tile)
+    return basis, pts, wts, ctx
+
+
+def _bound(precision, V):
+    return 1e-11 if precision == "fp64" else 1e-7 * np.abs(V).max()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32cache"])
+@pytest.mark.parametrize("method", ["svwn5", "pbe", "tpss"])
+@pytest.mark.parametrize("system,basis_name,tile", [
+    ("water", "6-31g", 0), ("water", "def2-svp", 0), ("methane", "6-31g(d,p)", 32),
+    ("water3", "def2-svp", 64), ("water3", "def2-tzvp", 0), ("alkane5", "def2-svp", 96),
+    ("alkane5", "6-31g", 0)])
+def test_build_matches_oracle(system, basis_name, tile, method, precision):
+    basis, pts, wts, ctx = _setup(system, basis_name, method, precision, tile)
+    D = random_density(basis.nbf, 5, 17)
+    K, exc, nel = oracle.xc_build(oracle.OracleBasis.from_flat(basis.flat()), pts, wts,
+                                  functional_ids(method), D)
+    for _ in range(2):
+        V, e, n = ctx.build(D)
+        assert np.abs(V - K).max() <= _bound(precision, K)
+        assert abs(e - exc) <= (1e-11 if precision == "fp64" else 1e-6)
+        assert abs(n - nel) <= (1e-11 if precision == "fp64" else 1e-6)
+    ctx.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32cache"])
+@pytest.mark.parametrize("method", ["svwn5", "blyp", "tpss"])
+@pytest.mark.parametrize("system,basis_name,tile", [
+    ("water", "6-31g", 0), ("methane", "def2-svp", 32), ("water3", "def2-tzvp", 0),
+    ("alkane5", "def2-svp", 64)])
+def test_unrestricted_build_matches_oracle(system, basis_name, tile, method, precision):
+    basis, pts, wts, ctx = _setup(system, basis_name, method, precision, tile)
+    # each spin block is read in full: an unsymmetric perturbation enters as it is
+    r = np.random.default_rng(3)
+    D = np.concatenate([random_density(basis.nbf, 5, 21), random_density(basis.nbf, 4, 22)]) / 2
+    if method != "tpss":
+        D = D + 1e-3 * r.normal(size=D.shape) * np.abs(D)
+    D = np.asfortranarray(D)
+    K, exc, nel = oracle.xc_build_unrestricted(oracle.OracleBasis.from_flat(basis.flat()), pts,
+                                               wts, functional_ids(method), D)
+    V, e, n = ctx.build_unrestricted(D)
+    assert np.abs(V - K).max() <= _bound(precision, K)
+    assert abs(e - exc) <= (1e-11 if precision == "fp64" else 1e-6)
+    assert np.abs(np.array(n) - np.array(nel)).max() <= (1e-11 if precision == "fp64" else 1e-6)
+    ctx.close()
