@@ -894,14 +894,9 @@ static void mgga_density(occxc_context *c, hipStream_t s) {
   const int prec = c->opt.precision;
   BuildArgs x = a;
   x.rho_out = c->d_mrho.get();
-  run_density_store(x, c->d_ao.get(), prec, c->d_D2.get(), s);
-  for (int k = 0; k < 3; ++k) {
-    BuildArgs y = a;
-    y.deriv = 0;
-    y.leaves = c->d_leaves_k.get() + (size_t)k * c->nleaves;
-    y.rho_out = c->d_mtau.get() + (size_t)k * c->ptot;
-    run_density_store(y, c->d_ao.get(), prec, c->d_D2.get(), s);
-  }
+  run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2.get(), s);
+  x.rho_out = c->d_mtau.get();
+  run_tau_store(c->plan, x, c->d_leaves_k.get(), c->d_ao.get(), prec, c->d_D2.get(), s);
   launch_functional_mgga_leaves(a, c->d_mrho.get(), c->d_mtau.get(), c->d_coef_tau.get(), s);
 }
 
@@ -984,7 +979,7 @@ static void run_nlc(occxc_context *c, const double *d_D, double b, double C, dou
   t.run(OCCXC_STAGE_DENSITY, [&] {
     BuildArgs x = a;
     x.rho_out = c->d_mrho.get();
-    run_density_store(x, c->d_ao.get(), prec, c->d_D2.get(), s);
+    run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2.get(), s);
   });
   t.run(OCCXC_STAGE_NLC, [&] {
     launch_vv10(a, c->d_mrho.get(), c->d_porig.get(), b, C, c->d_nlc.get(), c->npts, s);
@@ -1113,19 +1108,15 @@ static void mgga_density_u(occxc_context *c, hipStream_t s) {
   const BuildArgs &a = c->args;
   const int prec = c->opt.precision;
   const double *D2[2] = {c->d_D2a.get(), c->d_D2b.get()};
+  const double *D2s[2] = {c->d_D2sa.get(), c->d_D2sb.get()};
   double *rho[2] = {c->d_rho_a.get(), c->d_rho_b.get()};
   double *tk[2] = {c->d_mtau.get(), c->d_mtau_b.get()};
   for (int sp = 0; sp < 2; ++sp) {
     BuildArgs x = a;
     x.rho_out = rho[sp];
-    run_density_store(x, c->d_ao.get(), prec, D2[sp], s);
-    for (int k = 0; k < 3; ++k) {
-      BuildArgs y = a;
-      y.deriv = 0;
-      y.leaves = c->d_leaves_k.get() + (size_t)k * c->nleaves;
-      y.rho_out = tk[sp] + (size_t)k * c->ptot;
-      run_density_store(y, c->d_ao.get(), prec, D2[sp], s);
-    }
+    run_density_store(c->plan, x, c->d_ao.get(), prec, D2[sp], s);
+    x.rho_out = tk[sp];
+    run_tau_store(c->plan, x, c->d_leaves_k.get(), c->d_ao.get(), prec, D2s[sp], s);
   }
   launch_functional_mgga_pol_leaves(a, rho[0], rho[1], tk[0], tk[1], c->d_coef_b.get(),
                                     c->d_coef_tau.get(), c->d_coef_tau_b.get(),
@@ -1138,7 +1129,8 @@ void run_build_u(occxc_context *c, hipStream_t s) {
   const bool two_pass = c->plan.two_pass;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->nbf, s);
+    launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
+                             c->d_D2sb.get(), c->nbf, s);
     if (!two_pass) {
       launch_zero(c->d_K.get(), c->mtot, s);
       launch_zero(c->d_K_b.get(), c->mtot, s);
@@ -1161,9 +1153,9 @@ void run_build_u(occxc_context *c, hipStream_t s) {
   t.run(OCCXC_STAGE_DENSITY, [&] {
     BuildArgs x = a;
     x.rho_out = c->d_rho_a.get();
-    run_density_store(x, c->d_ao.get(), prec, c->d_D2a.get(), s);
+    run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2a.get(), s);
     x.rho_out = c->d_rho_b.get();
-    run_density_store(x, c->d_ao.get(), prec, c->d_D2b.get(), s);
+    run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2b.get(), s);
     launch_functional_pol_leaves(a, c->d_rho_a.get(), c->d_rho_b.get(), c->d_coef_b.get(),
                                  c->d_part_u.get(), s);
   });
@@ -1197,7 +1189,8 @@ void run_gradient_u(occxc_context *c, double *d_grad, hipStream_t s) {
   const int prec = c->opt.precision;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->nbf, s);
+    launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
+                             c->d_D2sb.get(), c->nbf, s);
   });
   if (c->mgga) {
     // process_grid_block_gradient<2, Unrestricted>: the unrestricted
@@ -1227,9 +1220,9 @@ void run_gradient_u(occxc_context *c, double *d_grad, hipStream_t s) {
   t.run(OCCXC_STAGE_DENSITY, [&] {
     BuildArgs x = a;
     x.rho_out = c->d_rho_a.get();
-    run_density_store(x, c->d_ao.get(), prec, c->d_D2a.get(), s);
+    run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2a.get(), s);
     x.rho_out = c->d_rho_b.get();
-    run_density_store(x, c->d_ao.get(), prec, c->d_D2b.get(), s);
+    run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2b.get(), s);
     launch_functional_pol_leaves(a, c->d_rho_a.get(), c->d_rho_b.get(), c->d_coef_b.get(),
                                  c->d_part_u.get(), s);
   });
@@ -1263,7 +1256,9 @@ void uks_setup(occxc_context *c) {
   if (c->mgga) {
     c->d_mtau_b.alloc(3 * (size_t)c->ptot);
     c->d_coef_tau_b.alloc(c->ptot);
-    c->device_bytes += 8.0 * 4 * (size_t)c->ptot;
+    c->d_D2sa.alloc(nn);
+    c->d_D2sb.alloc(nn);
+    c->device_bytes += 8.0 * (4 * (size_t)c->ptot + 2 * nn);
   }
   c->uks_ready = true;
 }

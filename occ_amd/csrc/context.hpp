@@ -91,8 +91,8 @@ struct occxc_context {
   bool mgga = false;
   occxc::DevBuf<double> d_mrho, d_mtau, d_coef_tau;
   // unrestricted meta-GGA: the beta spin's tau passes and c_tau (alpha uses
-  // d_mtau / d_coef_tau)
-  occxc::DevBuf<double> d_mtau_b, d_coef_tau_b;
+  // d_mtau / d_coef_tau), and D_s + D_s^T per spin for the tau passes
+  occxc::DevBuf<double> d_mtau_b, d_coef_tau_b, d_D2sa, d_D2sb;
   occxc::DevBuf<occxc::LeafDev> d_leaves_k;
   // VV10 (allocated on the first call): input-order point planes and F, U, W
   occxc::DevBuf<double> d_nlc;

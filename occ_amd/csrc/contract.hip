@@ -1584,12 +1584,15 @@ __device__ __forceinline__ void den_epi_first_loads(const S *__restrict__ ao, co
   }
 }
 
-template <typename S, bool GGA, bool PRE = false>
+// STORE: the sums of a leaf's only item go to a.rho_out (planes of ptot
+// doubles) instead of the functional; kq is the first quantity's plane there
+// and in the partial slots.
+template <typename S, bool GGA, bool PRE = false, bool STORE = false>
 __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *__restrict__ ao,
                                                   const DenItem &it, const LeafDev &L,
                                                   d4 (&acc)[4][4], double *__restrict__ part,
                                                   double *s_phi, double *s_red,
-                                                  const DenEpiFirst<S> *pre = nullptr) {
+                                                  const DenEpiFirst<S> *pre = nullptr, int kq = 0) {
   double(*s_q)[kMaxLeafPts] = reinterpret_cast<double(*)[kMaxLeafPts]>(s_phi);
   double(*s_h)[kTileAo] = reinterpret_cast<double(*)[kTileAo]>(s_phi + 4 * kMaxLeafPts);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1676,7 +1679,12 @@ __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *_
   }
   __syncthreads();
   const int nq = GGA ? 4 : 1;
-  if (it.part < 0) {
+  if (STORE && it.part < 0) {
+    for (int u = t; u < nq * it.np; u += 256) {
+      const int k = u / it.np, p = u - k * it.np;
+      a.rho_out[(kq + k) * a.ptot + L.pt_off + it.p0 + p] = s_q[k][p] + s_h[k][p];
+    }
+  } else if (it.part < 0) {
     // the leaf's only item: its points are the leaf's points
     for (int u = t; u < nq * it.np; u += 256) {
       const int k = u / it.np, p = u - k * it.np;
@@ -1690,7 +1698,7 @@ __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *_
     double *dst = part + (long long)it.part * 4 * kTileAo;
     for (int u = t; u < nq * it.np; u += 256) {
       const int k = u / it.np, p = u - k * it.np;
-      dst[k * kTileAo + p] = s_q[k][p] + s_h[k][p];
+      dst[(kq + k) * kTileAo + p] = s_q[k][p] + s_h[k][p];
     }
   }
 }
@@ -1821,13 +1829,22 @@ __device__ __forceinline__ void vmcnt_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <typename S, bool GGA>
+// SYM (LDA form, symmetric D2): only the row sums of (Phi D2) o Phi are
+// wanted, so the k-loop of column block [c0, c0 + wc) stops at the block's end
+// and the AOs before the block count twice: (nb - 1) / 2 nb of the MFMAs and of
+// the loads of a leaf of nb blocks go.
+// plane: the AO plane in Phi's place (1..3: the meta-GGA's tau passes, LDA
+// form), its sums going to quantity kq of the stored planes.
+template <typename S, bool GGA, bool SYM, bool STORE>
 __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *__restrict__ ao,
                                                   const int *__restrict__ ao_map,
                                                   const DenItem &it, double *__restrict__ part,
-                                                  char *s_stage, double *s_red) {
+                                                  char *s_stage, double *s_red, int plane = 0,
+                                                  int kq = 0) {
+  static_assert(!(GGA && SYM), "grad rho needs all of Phi D2");
   using P = DenDma<S>;
-  const LeafDev L = a.leaves[it.leaf];
+  LeafDev L = a.leaves[it.leaf];
+  if constexpr (STORE && !GGA) L.ao_off += (long long)plane * L.mp * L.np;
   const MolDev MD = a.mols[L.mol];
   const int t = threadIdx.x, lane = t & 63;
   // the wavefront index as a scalar: the AO rows of a load and their map
@@ -1894,7 +1911,8 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
     for (int j = 0; j < 4; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   // AO chunks up to the leaf's real AOs (the padding rows of Phi are zero);
   // the wavefront's tiles that hold real points and real AO columns
-  const int nch = (L.m + kTKc - 1) / kTKc;
+  const int nch = ((SYM ? min(L.m, it.c0 + it.wc) : L.m) + kTKc - 1) / kTKc;
+  const int cdbl = SYM && it.c0 > 0 ? it.c0 / kTKc : -1;  // first chunk of the block itself
   const int RTl = live_tiles(L.n - (it.p0 + wp * hp), hp), CTl = live_tiles(L.m - (it.c0 + wc * hc), hc);
   DenEpiFirst<S> pre;
   for (int c = 0; c < P::NS - 1 && c < nch; ++c) dma(c * kTKc, s_stage + c * P::STAGE);
@@ -1918,6 +1936,12 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
       const char *buf = s_stage + cur * P::STAGE;
       const S *sp = reinterpret_cast<const S *>(buf);
       const double *sd = reinterpret_cast<const double *>(buf + P::PHI);
+      if (SYM && c == cdbl) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+          for (int j = 0; j < NC; ++j) acc[i][j] *= 2.0;
+      }
       if constexpr (NR > 0)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
@@ -1936,15 +1960,22 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
       cur = cur + 1 == P::NS ? 0 : cur + 1;
     }
   });
-  den_tile_epilogue<S, GGA, true>(a, ao, it, L, acc, part, reinterpret_cast<double *>(s_stage),
-                                  s_red, &pre);
+  den_tile_epilogue<S, GGA, true, STORE>(a, ao, it, L, acc, part,
+                                         reinterpret_cast<double *>(s_stage), s_red, &pre, kq);
 }
 
-template <typename S, bool GGA>
+// The density items (STORE = false: restricted, D2 symmetric).  STORE: rho (and
+// grad rho, GGA) to a.rho_out; with the LDA form blockIdx.y + plane0 is the AO
+// plane, so that the three tau passes are one launch.  On (H2O)32 / def2-SVP
+// (FP64) the stored rho and grad rho of one spin take 2.95 ms where the
+// per-leaf k_density_wave took 5.2, the three tau passes 5.3 ms (4.2e9 bytes
+// of plane each read once for the k-loop and once for the row sums; without
+// SYM's shorter k-loop 20 to 30 % more MFMAs) where it took 12.7.
+template <typename S, bool GGA, bool SYM, bool STORE>
 __global__ __launch_bounds__(256, 2) void k_den_tile_dma(BuildArgs a, const S *__restrict__ ao,
                                                          const int *__restrict__ ao_map,
                                                          const DenItem *__restrict__ items,
-                                                         double *__restrict__ part) {
+                                                         double *__restrict__ part, int plane0) {
   // one LDS array (the reduction slots after the chunk buffers): with a
   // second __shared__ variable the LDS accesses carry alias scopes, and the
   // compiler then waits for every direct load in flight before each chunk's
@@ -1953,7 +1984,8 @@ __global__ __launch_bounds__(256, 2) void k_den_tile_dma(BuildArgs a, const S *_
   double *s_red = reinterpret_cast<double *>(s_stage + DenDma<S>::NS * DenDma<S>::STAGE);
   const DenItem it = items[blockIdx.x];
   if (it.leaf < 0) return;
-  den_tile_item_dma<S, GGA>(a, ao, ao_map, it, part, s_stage, s_red);
+  den_tile_item_dma<S, GGA, SYM, STORE>(a, ao, ao_map, it, part, s_stage, s_red,
+                                        plane0 + blockIdx.y, blockIdx.y);
 }
 
 // PERSIST: the workgroups loop over the items blockIdx.x, blockIdx.x +
@@ -2003,6 +2035,22 @@ __global__ __launch_bounds__(256) void k_den_finish(BuildArgs a, const DenFinish
   }
   __syncthreads();
   density_epilogue(a, L, F.leaf, s_q, s_red);
+}
+
+// The same sums (nq quantities) to a.rho_out, without the functional.
+__global__ __launch_bounds__(256) void k_den_finish_store(BuildArgs a,
+                                                           const DenFinish *__restrict__ fin,
+                                                           const double *__restrict__ part, int nq) {
+  const DenFinish F = fin[blockIdx.x];
+  const LeafDev L = a.leaves[F.leaf];
+  for (int u = threadIdx.x; u < nq * L.np; u += blockDim.x) {
+    const int k = u / L.np, p = u - k * L.np;
+    const int pb = p / kTileAo, pl = p - pb * kTileAo;
+    const double *src = part + (long long)(F.part0 + pb * F.ncb) * 4 * kTileAo + k * kTileAo + pl;
+    double v = 0.0;
+    for (int cb = 0; cb < F.ncb; ++cb) v += src[(long long)cb * 4 * kTileAo];
+    a.rho_out[k * a.ptot + L.pt_off + p] = v;
+  }
 }
 
 // Scatter of a Vxc item's block into K with FP64 atomics (entries below cut
@@ -3107,9 +3155,28 @@ ContractPlan make_contract_plan(const std::vector<LeafDev> &leaves, long long mt
   return p;
 }
 
-void run_density_store(const BuildArgs &a, const void *ao, int precision, const double *D2t,
-                       hipStream_t s) {
+void run_density_store(const ContractPlan &plan, const BuildArgs &a, const void *ao,
+                       int precision, const double *D2t, hipStream_t s) {
   if (a.nleaves == 0) return;
+  if (plan.tiled && plan.den_dma) {
+    auto launch = [&](auto s_tag) {
+      using S = decltype(s_tag);
+      BuildArgs x = a;
+      x.D2 = D2t;
+      (a.deriv ? k_den_tile_dma<S, true, false, true> : k_den_tile_dma<S, false, false, true>)
+          <<<plan.n_den_items, 256, 0, s>>>(x, static_cast<const S *>(ao), a.ao_map,
+                                            plan.den_items.get(), plan.den_part.get(), 0);
+    };
+    if (precision == 0) launch(double{});
+    else launch(float{});
+    check_launch("k_den_tile_dma (store)");
+    if (plan.n_den_finish > 0) {
+      k_den_finish_store<<<plan.n_den_finish, 256, 0, s>>>(a, plan.den_finish.get(),
+                                                           plan.den_part.get(), a.deriv ? 4 : 1);
+      check_launch("k_den_finish_store");
+    }
+    return;
+  }
   if (precision == 0)
     k_density_wave<double, double, true>
         <<<a.nleaves, 256, 0, s>>>(a, static_cast<const double *>(ao), D2t, 0);
@@ -3117,6 +3184,36 @@ void run_density_store(const BuildArgs &a, const void *ao, int precision, const 
     k_density_wave<float, double, true>
         <<<a.nleaves, 256, 0, s>>>(a, static_cast<const float *>(ao), D2t, 0);
   check_launch("k_density_wave (store)");
+}
+
+void run_tau_store(const ContractPlan &plan, const BuildArgs &a, const LeafDev *leaves_k,
+                   const void *ao, int precision, const double *D2s, hipStream_t s) {
+  if (a.nleaves == 0) return;
+  if (plan.tiled && plan.den_dma) {
+    auto launch = [&](auto s_tag) {
+      using S = decltype(s_tag);
+      BuildArgs x = a;
+      x.D2 = D2s;
+      k_den_tile_dma<S, false, true, true><<<dim3(plan.n_den_items, 3), 256, 0, s>>>(
+          x, static_cast<const S *>(ao), a.ao_map, plan.den_items.get(), plan.den_part.get(), 1);
+    };
+    if (precision == 0) launch(double{});
+    else launch(float{});
+    check_launch("k_den_tile_dma (tau)");
+    if (plan.n_den_finish > 0) {
+      k_den_finish_store<<<plan.n_den_finish, 256, 0, s>>>(a, plan.den_finish.get(),
+                                                           plan.den_part.get(), 3);
+      check_launch("k_den_finish_store (tau)");
+    }
+    return;
+  }
+  for (int k = 0; k < 3; ++k) {
+    BuildArgs y = a;
+    y.deriv = 0;
+    y.leaves = leaves_k + (size_t)k * a.nleaves;
+    y.rho_out = a.rho_out + (size_t)k * a.ptot;
+    run_density_store(plan, y, ao, precision, D2s, s);
+  }
 }
 
 void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, int precision,
@@ -3132,9 +3229,9 @@ void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, i
             <<<std::min(2 * plan.persistent_wgs, plan.n_den_items), 256, 0, s>>>(
                 a, x, plan.den_items.get(), plan.den_part.get(), plan.n_den_items);
       else if (plan.den_dma)
-        (a.deriv ? k_den_tile_dma<S, true> : k_den_tile_dma<S, false>)
+        (a.deriv ? k_den_tile_dma<S, true, false, false> : k_den_tile_dma<S, false, true, false>)
             <<<plan.n_den_items, 256, 0, s>>>(a, x, a.ao_map, plan.den_items.get(),
-                                              plan.den_part.get());
+                                              plan.den_part.get(), 0);
       else
         (a.deriv ? k_den_tile<S, true> : k_den_tile<S, false>)
             <<<plan.n_den_items, 256, 0, s>>>(a, x, plan.den_items.get(), plan.den_part.get(),

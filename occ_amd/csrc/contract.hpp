@@ -76,8 +76,12 @@ void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, i
                  hipStream_t s);
 // rho and grad rho of every leaf point for the density D2t into a.rho_out
 // (FP64 or FP32-cache contexts, leaves of at most 2048 AOs)
-void run_density_store(const BuildArgs &a, const void *ao, int precision, const double *D2t,
-                       hipStream_t s);
+void run_density_store(const ContractPlan &plan, const BuildArgs &a, const void *ao,
+                       int precision, const double *D2t, hipStream_t s);
+// meta-GGA: rowsum((d_k Phi D2s) o d_k Phi) of the three directions into
+// a.rho_out ([3][ptot]); D2s must be symmetric.  leaves_k as run_vxc_mgga's.
+void run_tau_store(const ContractPlan &plan, const BuildArgs &a, const LeafDev *leaves_k,
+                   const void *ao, int precision, const double *D2s, hipStream_t s);
 constexpr int kStoreMaxMp = 2048;
 void run_vxc(const ContractPlan &plan, const BuildArgs &a, const void *ao, int precision,
              hipStream_t s);

@@ -552,15 +552,22 @@ __global__ void k_prepare_density(const double *__restrict__ D, double *__restri
 // Unrestricted D (2 nbf x nbf, alpha rows over beta rows, one molecule):
 // D2t_s = 2 D_s^T for each spin, the full block (evaluate_density<d, U> uses
 // no selfadjointView, density.cpp:18-30,45-70); the contraction kernels read
-// D2t(nu, mu) as D2(mu, nu).
+// D2t(nu, mu) as D2(mu, nu).  D2sa / D2sb (null unless a meta-GGA): D_s + D_s^T,
+// exactly symmetric, which gives the tau row sums of 2 D_s.
 __global__ void k_prepare_density_u(const double *__restrict__ D, double *__restrict__ D2a,
-                                    double *__restrict__ D2b, int nbf) {
+                                    double *__restrict__ D2b, double *__restrict__ D2sa,
+                                    double *__restrict__ D2sb, int nbf) {
   const long long n = (long long)nbf * nbf;
   for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n;
        k += (long long)gridDim.x * blockDim.x) {
     const int nu = (int)(k % nbf), mu = (int)(k / nbf);
-    D2a[k] = 2.0 * D[mu + (long long)nu * 2 * nbf];
-    D2b[k] = 2.0 * D[nbf + mu + (long long)nu * 2 * nbf];
+    const double da = D[mu + (long long)nu * 2 * nbf], db = D[nbf + mu + (long long)nu * 2 * nbf];
+    D2a[k] = 2.0 * da;
+    D2b[k] = 2.0 * db;
+    if (D2sa) {
+      D2sa[k] = da + D[nu + (long long)mu * 2 * nbf];
+      D2sb[k] = db + D[nbf + nu + (long long)mu * 2 * nbf];
+    }
   }
 }
 
@@ -1166,11 +1173,11 @@ void launch_finalize_scalars(const MolDev *mols, int nmol, const double *leaf_pa
   check_launch();
 }
 
-void launch_prepare_density_u(const double *D, double *D2a, double *D2b, int nbf,
-                              hipStream_t s) {
+void launch_prepare_density_u(const double *D, double *D2a, double *D2b, double *D2sa,
+                              double *D2sb, int nbf, hipStream_t s) {
   const long long n = (long long)nbf * nbf;
   if (n == 0) return;
-  k_prepare_density_u<<<grid_for(n, 256), 256, 0, s>>>(D, D2a, D2b, nbf);
+  k_prepare_density_u<<<grid_for(n, 256), 256, 0, s>>>(D, D2a, D2b, D2sa, D2sb, nbf);
   check_launch();
 }
 

@@ -244,12 +244,13 @@ void launch_xc_gradient(const BuildArgs &a, const void *ao, bool ao_fp32, const 
 void launch_density_functional(const BuildArgs &a, const void *ao, bool fp32,
                                hipStream_t s);
 void launch_vxc(const BuildArgs &a, const void *ao, bool fp32, hipStream_t s);
-// unrestricted build (one molecule): D2t_s = 2 D_s^T; the polarised
+// unrestricted build (one molecule): D2t_s = 2 D_s^T and, when D2sa is given
+// (meta-GGA), D_s + D_s^T per spin; the polarised
 // functional stage per leaf (coef_a in a.coef, {Exc, N_a, N_b} per leaf in
 // part); V_s = K_s + K_s^T (skipped when Ka is null) and the fixed-order
 // scalar sums into result[3]
-void launch_prepare_density_u(const double *D, double *D2a, double *D2b, int nbf,
-                              hipStream_t s);
+void launch_prepare_density_u(const double *D, double *D2a, double *D2b, double *D2sa,
+                              double *D2sb, int nbf, hipStream_t s);
 void launch_functional_pol_leaves(const BuildArgs &a, const double *rho_a, const double *rho_b,
                                   double *coef_b, double *part, hipStream_t s);
 void launch_finalize_u(const double *Ka, const double *Kb, double *Va, double *Vb,

@@ -67,9 +67,7 @@ def test_unrestricted_build_matches_oracle(system, basis_name, tile, method, pre
     # each spin block is read in full: an unsymmetric perturbation enters as it is
     r = np.random.default_rng(3)
     D = np.concatenate([random_density(basis.nbf, 5, 21), random_density(basis.nbf, 4, 22)]) / 2
-    if method != "tpss":
-        D = D + 1e-3 * r.normal(size=D.shape) * np.abs(D)
-    D = np.asfortranarray(D)
+    D = np.asfortranarray(D + 1e-3 * r.normal(size=D.shape) * np.abs(D))
     K, exc, nel = oracle.xc_build_unrestricted(oracle.OracleBasis.from_flat(basis.flat()), pts,
                                                wts, functional_ids(method), D)
     V, e, n = ctx.build_unrestricted(D)
