@@ -1024,11 +1024,11 @@ void gradient_setup(occxc_context *c, int natoms, const int *shell_atom) {
     const size_t n = c->ao_elems / c->ncomp * (c->deriv ? 6 : 3);
     c->d_ao2.alloc(std::max<size_t>(n, 1));
     c->d_gpart.alloc(std::max<size_t>(3 * c->d_ao_map.size(), 1));
-    c->device_bytes += c->d_ao2.bytes() + c->d_gpart.bytes();
-    if (c->mgga) {
-      c->d_gpart2.alloc(c->d_gpart.size());
-      c->device_bytes += c->d_gpart2.bytes();
-    }
+    const auto items = gradient_items(c->leaves, c->mgga ? kGradWideTau : kGradWide);
+    c->n_gitems = (int)items.size();
+    c->d_gitems.alloc(std::max<size_t>(items.size(), 1));
+    c->d_gitems.upload(items.data(), items.size(), c->stream);
+    c->device_bytes += c->d_ao2.bytes() + c->d_gpart.bytes() + c->d_gitems.bytes();
     StageTimer t{c, c->stream, {}};
     t.run(OCCXC_STAGE_AO,
           [&] { launch_ao_extra(c->args, c->d_ao2.get(), c->deriv != 0, c->stream); });
@@ -1054,6 +1054,7 @@ void gradient_setup(occxc_context *c, int natoms, const int *shell_atom) {
   c->d_gatom_ent.alloc(ent.size());
   c->d_gatom_ent.upload(ent.data(), ent.size(), c->stream);
   c->d_grad.alloc(3 * (size_t)natoms);
+  c->d_gred.alloc(3 * (size_t)kGradSplit * natoms);
   OCCXC_HIP(hipStreamSynchronize(c->stream));
   c->grad_shell_atom.assign(shell_atom, shell_atom + c->nsh);
   c->grad_natoms = natoms;
@@ -1067,32 +1068,27 @@ void run_gradient(occxc_context *c, const double *d_D, double *d_grad, hipStream
   t.run(OCCXC_STAGE_PREPARE, [&] {
     launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf, s);
   });
-  if (c->mgga) {
-    // process_grid_block_gradient<2, Restricted>: the meta-GGA density stage,
-    // the GGA terms and the tau terms as two partial sets, one reduction
-    const bool fp32 = c->opt.precision != OCCXC_PREC_FP64;
-    t.run(OCCXC_STAGE_DENSITY, [&] { mgga_density(c, s); });
-    t.run(OCCXC_STAGE_GRADIENT, [&] {
-      launch_xc_gradient_partials(a, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart.get(), s);
-      BuildArgs x = a;
-      x.coef_tau = c->d_coef_tau.get();
-      x.coef_tau_planes = 1;
-      launch_xc_gradient_tau(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart2.get(), s);
-      launch_grad_reduce(c->d_gpart.get(), c->d_gpart2.get(), c->grad_natoms,
-                         c->d_gatom_off.get(), c->d_gatom_ent.get(), d_grad, s);
-    });
-    return;
-  }
   t.run(OCCXC_STAGE_DENSITY, [&] {
-    if (c->plan.use_mfma)
+    if (c->mgga)
+      mgga_density(c, s);
+    else if (c->plan.use_mfma)
       run_density(c->plan, a, c->d_ao.get(), c->opt.precision, s);
     else
       launch_density_functional(a, c->d_ao.get(), c->opt.precision != OCCXC_PREC_FP64, s);
   });
   t.run(OCCXC_STAGE_GRADIENT, [&] {
-    launch_xc_gradient(a, c->d_ao.get(), c->opt.precision != OCCXC_PREC_FP64, c->d_ao2.get(),
-                       c->d_gpart.get(), c->grad_natoms, c->d_gatom_off.get(),
-                       c->d_gatom_ent.get(), d_grad, s);
+    // process_grid_block_gradient<d, Restricted>; the tau terms of a meta-GGA
+    // come with a.coef_tau
+    BuildArgs x = a;
+    if (c->mgga) {
+      x.coef_tau = c->d_coef_tau.get();
+      x.coef_tau_planes = 1;
+    }
+    launch_xc_gradient_partials(x, c->d_ao.get(), c->opt.precision != OCCXC_PREC_FP64,
+                                c->d_ao2.get(), c->d_gitems.get(), c->n_gitems,
+                                c->d_gpart.get(), s);
+    launch_grad_reduce(c->d_gpart.get(), nullptr, c->grad_natoms, c->d_gatom_off.get(),
+                       c->d_gatom_ent.get(), c->d_gred.get(), d_grad, s);
   });
 }
 
@@ -1192,32 +1188,11 @@ void run_gradient_u(occxc_context *c, double *d_grad, hipStream_t s) {
     launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
                              c->d_D2sb.get(), c->nbf, s);
   });
-  if (c->mgga) {
-    // process_grid_block_gradient<2, Unrestricted>: the unrestricted
-    // meta-GGA density stage, per spin the GGA and tau partial sets, one
-    // reduction of all four
-    const bool fp32 = prec != OCCXC_PREC_FP64;
-    t.run(OCCXC_STAGE_DENSITY, [&] { mgga_density_u(c, s); });
-    t.run(OCCXC_STAGE_GRADIENT, [&] {
-      BuildArgs x = a;
-      x.D2 = c->d_D2a.get();
-      x.coef_tau = c->d_coef_tau.get();
-      x.coef_tau_planes = 1;
-      launch_xc_gradient_partials(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart.get(), s);
-      launch_xc_gradient_tau(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart3.get(), s);
-      x.D2 = c->d_D2b.get();
-      x.coef = c->d_coef_b.get();
-      x.coef_tau = c->d_coef_tau_b.get();
-      x.coef_tau_planes = 1;
-      launch_xc_gradient_partials(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart2.get(), s);
-      launch_xc_gradient_tau(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart4.get(), s);
-      launch_grad_reduce(c->d_gpart.get(), c->d_gpart2.get(), c->grad_natoms,
-                         c->d_gatom_off.get(), c->d_gatom_ent.get(), d_grad, s,
-                         c->d_gpart3.get(), c->d_gpart4.get());
-    });
-    return;
-  }
   t.run(OCCXC_STAGE_DENSITY, [&] {
+    if (c->mgga) {
+      mgga_density_u(c, s);
+      return;
+    }
     BuildArgs x = a;
     x.rho_out = c->d_rho_a.get();
     run_density_store(c->plan, x, c->d_ao.get(), prec, c->d_D2a.get(), s);
@@ -1227,15 +1202,26 @@ void run_gradient_u(occxc_context *c, double *d_grad, hipStream_t s) {
                                  c->d_part_u.get(), s);
   });
   t.run(OCCXC_STAGE_GRADIENT, [&] {
+    // per spin one partial set (with the tau terms of a meta-GGA), one
+    // reduction of both
     const bool fp32 = prec != OCCXC_PREC_FP64;
-    BuildArgs x = a;
-    x.D2 = c->d_D2a.get();
-    launch_xc_gradient_partials(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart.get(), s);
-    x.D2 = c->d_D2b.get();
-    x.coef = c->d_coef_b.get();
-    launch_xc_gradient_partials(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gpart2.get(), s);
-    launch_grad_reduce(c->d_gpart.get(), c->d_gpart2.get(), c->grad_natoms,
-                       c->d_gatom_off.get(), c->d_gatom_ent.get(), d_grad, s);
+    const double *D2[2] = {c->d_D2a.get(), c->d_D2b.get()};
+    double *coef[2] = {a.coef, c->d_coef_b.get()};
+    const double *ct[2] = {c->d_coef_tau.get(), c->d_coef_tau_b.get()};
+    double *gp[2] = {c->d_gpart.get(), c->d_gpart2.get()};
+    for (int sp = 0; sp < 2; ++sp) {
+      BuildArgs x = a;
+      x.D2 = D2[sp];
+      x.coef = coef[sp];
+      if (c->mgga) {
+        x.coef_tau = ct[sp];
+        x.coef_tau_planes = 1;
+      }
+      launch_xc_gradient_partials(x, c->d_ao.get(), fp32, c->d_ao2.get(), c->d_gitems.get(),
+                                  c->n_gitems, gp[sp], s);
+    }
+    launch_grad_reduce(gp[0], gp[1], c->grad_natoms, c->d_gatom_off.get(),
+                       c->d_gatom_ent.get(), c->d_gred.get(), d_grad, s);
   });
 }
 
@@ -1629,11 +1615,6 @@ static void gradient_u_prepare(occxc_context *ctx, int natoms, const int *shell_
                     std::to_string(kStoreMaxMp) + " AOs");
   gradient_setup(ctx, natoms, shell_atom);
   uks_setup(ctx);
-  if (ctx->mgga && ctx->d_gpart3.size() < ctx->d_gpart.size()) {
-    ctx->d_gpart3.alloc(ctx->d_gpart.size());
-    ctx->d_gpart4.alloc(ctx->d_gpart.size());
-    ctx->device_bytes += ctx->d_gpart3.bytes() + ctx->d_gpart4.bytes();
-  }
   if (ctx->d_gpart2.size() < ctx->d_gpart.size()) {
     ctx->d_gpart2.alloc(ctx->d_gpart.size());
     ctx->device_bytes += ctx->d_gpart2.bytes();

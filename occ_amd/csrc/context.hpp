@@ -70,9 +70,9 @@ struct occxc_context {
   // per-AO partial sums, and the per-atom entry lists built for the
   // shell-to-atom map of the last call
   std::vector<int> bf_shell;
-  occxc::DevBuf<double> d_ao2, d_gpart, d_gpart2, d_grad;
-  // unrestricted meta-GGA gradient: each spin's tau partials
-  occxc::DevBuf<double> d_gpart3, d_gpart4;
+  occxc::DevBuf<double> d_ao2, d_gpart, d_gpart2, d_grad, d_gred;
+  occxc::DevBuf<occxc::DenItem> d_gitems;
+  int n_gitems = 0;
   occxc::DevBuf<int> d_gatom_off, d_gatom_ent;
   bool ao2_ready = false;
   std::vector<int> grad_shell_atom;

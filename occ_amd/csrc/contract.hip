@@ -29,6 +29,7 @@
 #include <string>
 
 #include "contract.hpp"
+#include "tile_dma.hpp"
 #include "tuning_table.hpp"
 #include "xc_functionals.hpp"
 
@@ -1481,10 +1482,6 @@ __device__ __forceinline__ void tile_shape(int rt, int ct, F &&f) {
 // Those kernels pass each wavefront's live tiles (live_tiles), and 0 runs
 // no MFMA.
 
-// 16-row tiles of a wavefront's half block (half rows) that hold any of the
-// `valid` rows counted from its first row: the tiles past a leaf's real AOs
-// or points hold padding only (zero AO rows, zero-weight points) and are not
-// computed.  One tile runs as the 2-tile shape (the shapes start at 2).
 template <typename F>
 __device__ __forceinline__ void tile_shape_ext(int rt, int ct, F &&f) {
   if (rt == 0 || ct == 0) f(IntC<0>{}, IntC<0>{});  // no tile: loads and barriers only
@@ -1497,11 +1494,6 @@ __device__ __forceinline__ void tile_shape_ext(int rt, int ct, F &&f) {
   else if (rt == 2 && ct == 3) f(IntC<2>{}, IntC<3>{});
   else if (rt == 2 && ct == 2) f(IntC<2>{}, IntC<2>{});
   else f(IntC<4>{}, IntC<4>{});
-}
-
-__device__ __forceinline__ int live_tiles(int valid, int half) {
-  const int t = (min(max(valid, 0), half) + 15) >> 4;
-  return t == 1 ? 2 : t;
 }
 
 // Two FP64 k-steps of acc[i][j] += X_i^T Y_j.  x and y point at this lane's
@@ -1816,18 +1808,6 @@ template <typename S> struct DenDma {
   static constexpr int LOADS = (sizeof(S) == 8 ? 4 : 2) + 16;     // loads per chunk per wavefront
 };
 static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float>::STAGE / 8, "epilogue sums fit a stage");
-
-// Barrier after this wavefront's vector memory loads but the newest N are
-// done (and its LDS accesses): the s_waitcnt immediate holds vmcnt in bits
-// 3:0 and 15:14, expcnt (no wait) in 6:4 and lgkmcnt (0) in 11:8.
-template <int N>
-__device__ __forceinline__ void vmcnt_barrier() {
-  static_assert(N >= 0 && N < 64, "vmcnt is six bits");
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | ((N >> 4) << 14));
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // SYM (LDA form, symmetric D2): only the row sums of (Phi D2) o Phi are
 // wanted, so the k-loop of column block [c0, c0 + wc) stops at the block's end
@@ -2524,17 +2504,6 @@ __global__ __launch_bounds__(256, 2) void k_vxc_gemm_f32(BuildArgs a, const floa
   vxc_scatter<true, true>(acc, it, L, MD, map, Km, kScatterCut, reinterpret_cast<double *>(s_stage));
 }
 
-// Workgroup barrier for LDS hand-offs only: waits for this wavefront's LDS
-// accesses (lgkmcnt) but not for its outstanding global memory operations,
-// so the MFMA wavefronts' scatter atomics drain while the next steps run
-// (__syncthreads would wait for them at every step).  The empty asm
-// statements keep the compiler from moving memory accesses across it.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // vmcnt and expcnt: no wait; lgkmcnt(0)
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 // Vxc item in FP64 (FP64 / FP32-cache contexts), block pair (r, c) of a leaf,
 // the raw AO planes staged by direct-to-LDS loads.  A chunk is 64 bytes of
 // every staged AO row and plane: vd_pts() points (8 with FP64 storage, 16 with
@@ -2986,11 +2955,37 @@ TuneChoice tune_choice(const occxc_options *opt, int max_nbf) {
   return t;
 }
 
+static constexpr int kXcdRuns = 8;
+// one list per XCD -> entry 8 k + x is the k-th of run x
+template <typename T>
+static std::vector<T> interleave_runs(const std::vector<std::vector<T>> &lists, T pad) {
+  size_t len = 0;
+  for (auto &l : lists) len = std::max(len, l.size());
+  std::vector<T> out(len * kXcdRuns, pad);
+  for (int x = 0; x < kXcdRuns; ++x)
+    for (size_t k = 0; k < lists[x].size(); ++k) out[k * kXcdRuns + x] = lists[x][k];
+  return out;
+}
+
+std::vector<DenItem> gradient_items(const std::vector<LeafDev> &leaves, int maxw) {
+  double total = 0.0, acc = 0.0;
+  for (const auto &L : leaves) total += (double)L.np * L.mp * L.mp;
+  std::vector<std::vector<DenItem>> lists(kXcdRuns);
+  for (int li = 0; li < (int)leaves.size(); ++li) {
+    const LeafDev &L = leaves[li];
+    const int x = std::min(kXcdRuns - 1, (int)(acc / std::max(total, 1.0) * kXcdRuns));
+    acc += (double)L.np * L.mp * L.mp;
+    for (const auto &b : tile_blocks(L.mp, maxw))
+      lists[x].push_back(DenItem{li, -1, 0, (short)L.np, (short)b.first, (short)b.second});
+  }
+  return interleave_runs(lists, DenItem{-1, -1, 0, 0, 0, 0});
+}
+
 // vxc_only: the Vxc item list alone (FP32 storage without the tiled build
 // kernels needs it once, for dS).
 static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
                            bool vxc_only = false) {
-  constexpr int kXcd = 8;
+  constexpr int kXcd = kXcdRuns;
   const int nl = (int)leaves.size();
   double total = 0.0;
   for (const auto &L : leaves) total += (double)L.np * L.mp * L.mp;
@@ -3019,16 +3014,8 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
         vxc[x].push_back(VxcItem{li, (short)cb[r].first, (short)cb[r].second,
                                  (short)cb[c].first, (short)cb[c].second, 0});
   }
-  auto interleave = [&](auto &lists, auto pad) {
-    size_t len = 0;
-    for (auto &l : lists) len = std::max(len, l.size());
-    std::vector<decltype(pad)> out(len * kXcd, pad);
-    for (int x = 0; x < kXcd; ++x)
-      for (size_t k = 0; k < lists[x].size(); ++k) out[k * kXcd + x] = lists[x][k];
-    return out;
-  };
-  const auto d = interleave(den, DenItem{-1, -1, 0, 0, 0, 0});
-  const auto v = interleave(vxc, VxcItem{-1, 0, 0, 0, 0, 0});
+  const auto d = interleave_runs(den, DenItem{-1, -1, 0, 0, 0, 0});
+  const auto v = interleave_runs(vxc, VxcItem{-1, 0, 0, 0, 0, 0});
   p.n_vxc_items = (int)v.size();
   p.vxc_items.alloc(std::max<size_t>(v.size(), 1));
   p.vxc_items.upload(v.data(), v.size());

@@ -56,6 +56,10 @@ struct ContractPlan {
 // one leaf (an upper bound used before the plan exists)
 double tile_plan_bytes(const LeafDev &L);
 
+// The gradient's items: every leaf's column blocks of at most maxw AOs
+// (all its points: p0 = 0, np), interleaved over the XCDs as the build's.
+std::vector<DenItem> gradient_items(const std::vector<LeafDev> &leaves, int maxw);
+
 // Vxc kernel selection (OCCXC_VXC_VARIANT, default 0)
 int vxc_variant_setting();
 

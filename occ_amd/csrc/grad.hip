@@ -13,292 +13,327 @@
 // gives the same number with two leaf GEMMs instead of three m x m ones:
 //   G(k, A) = -2 sum_{mu on A} sum_p [d_k phi_mu U_mu + aow_k,mu T_mu],
 //   T = Phi P (the density's own product), U = Aow P.
-// One workgroup per active leaf; each wavefront owns 32-AO chunks of the
-// leaf and, for each 32-point block, forms T and U on the FP64 matrix cores
-// (A operand Phi and Aow = c0 Phi + c . grad Phi built in registers, B operand
-// P gathered through the AO map), then adds the integrand into per-lane sums
-// of its AOs.  The per-AO sums go to gpart; a second kernel reduces them per
-// atom in a fixed order (no atomics: the gradient repeats bit for bit).
+// One workgroup per (leaf, column block of AOs): it walks the leaf's points 64
+// at a time, forms the products on the FP64 matrix cores from operands staged
+// by direct-to-LDS loads, and adds the integrand into per-lane sums of its
+// AOs.  The meta-GGA's tau terms (accumulate_gradient_contribution_R<2>,
+// dft_gradient_kernels.cpp:152-172),
+//   V_k += sum_j d_kj phi^T ((vtau / 2) d_j phi),
+// contract to sum_p sum_j d_kj phi_mu (vtau / 2) T_j,mu with T_j = (d_j Phi) P;
+// there U = c0 T + sum_j c_j T_j needs no product of its own.
+// The per-AO sums go to gpart; two more kernels reduce them per atom in a
+// fixed order (no atomics: the gradient repeats bit for bit).
 #include <hip/hip_runtime.h>
 
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 #include "kernels.hpp"
+#include "tile_dma.hpp"
 
 namespace occxc {
 
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ d4 mma(double a, double b, d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-template <typename S> __device__ __forceinline__ d4 load4d(const S *p);
-template <> __device__ __forceinline__ d4 load4d<double>(const double *p) {
-  return *reinterpret_cast<const d4 *>(p);
+template <typename S> __device__ __forceinline__ d2 load2d(const S *p);
+template <> __device__ __forceinline__ d2 load2d<double>(const double *p) {
+  return *reinterpret_cast<const d2 *>(p);
 }
-template <> __device__ __forceinline__ d4 load4d<float>(const float *p) {
-  const f4 v = *reinterpret_cast<const f4 *>(p);
-  return d4{(double)v[0], (double)v[1], (double)v[2], (double)v[3]};
+template <> __device__ __forceinline__ d2 load2d<float>(const float *p) {
+  const f2 v = *reinterpret_cast<const f2 *>(p);
+  return d2{(double)v[0], (double)v[1]};
 }
 
-// Same leaf order over the XCDs as the build's contraction kernels.
-__device__ __forceinline__ int xcd_leaf(int b, int n) {
-  constexpr int kXcd = 8;
-  const int x = b % kXcd, i = b / kXcd, q = n / kXcd, r = n % kXcd;
-  return x * q + min(x, r) + i;
+template <typename T> __device__ __forceinline__ const T *at(const T *base, unsigned bytes) {
+  return reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
 }
+
+// Staging of the gradient items.  A chunk is kGk AOs: their rows of the NQ
+// planes at the item's 64 points ([plane][AO][point], as stored) and of P,
+// gathered through the AO map ([AO][column], each double as two 4-byte pieces
+// from two lanes).  NT products: 1 (LDA: T), 2 (GGA: T and U) or 4 (meta-GGA:
+// T and the three T_j), 16 accumulator tiles a wavefront in all, so the
+// meta-GGA's column blocks are half as wide.  Three chunk buffers, two chunks
+// in flight; every wavefront issues the same number of loads for a chunk.
+// Bound by HBM: the nine derivative planes of the integrand are read once
+// (1.9e10 bytes on (H2O)32 / def2-SVP, FP64), the four of the products once per
+// column block.  PBE there 11.76 -> 6.70 ms against the per-leaf form, which
+// read the products' planes once per 32 AOs through each lane's own loads; the
+// TPSS terms of C11H24, 5.95 -> 2.53 ms for both spins (five products of two
+// kernels then, four of one now).
+constexpr int kGk = 8, kGp = kGradPoints;
+template <typename S, int NT> struct GradDma {
+  static constexpr int NS = 3;
+  static constexpr int NQ = NT == 1 ? 1 : 4;
+  static constexpr int CW = NT == 4 ? 64 : 128;              // widest column block
+  static constexpr int PLANE = kGk * kGp * (int)sizeof(S);   // bytes of a plane's rows
+  static constexpr int STAGE = NQ * PLANE + kGk * CW * 8;
+  static constexpr int PI = PLANE / 1024;                    // loads of a plane
+  static constexpr int PL = NQ == 4 ? PI : PI / 4 + (PI < 4);  // a wavefront's (LDA: shared out)
+  static constexpr int LOADS = PL + 2 * (CW / 32);
+  static constexpr int NC = NT == 1 ? 1 : NT == 2 ? 4 : 5;   // coefficient planes
+};
 
 // MFMA layout (v_mfma_f64_16x16x4f64): lane l supplies A[l%16][l/16] and
 // B[l/16][l%16]; accumulator register r of lane l holds row l/16 + 4r,
 // column l%16.  Point row i of a 16-point tile is fed as point
 // 4(i%4) + i/4, so lane group g's accumulator rows are the 4 consecutive
-// points 4g..4g+3 (vector loads in the integrand).  The contraction index
-// mu = mc + 4g + s (step s = 0..3) is any permutation shared by A and B.
-template <typename S, bool GGA>
-__global__ __launch_bounds__(256, 2) void k_xc_grad(BuildArgs a, const S *__restrict__ ao,
-                                                   const double *__restrict__ ao2,
-                                                   double *__restrict__ gpart) {
-  __shared__ double s_c[4][kMaxLeafPts];
-  const int leaf = xcd_leaf(blockIdx.x, gridDim.x);
-  const LeafDev L = a.leaves[leaf];
-  double *gp = gpart + 3LL * L.map_off;
-  if (!a.leaf_active[leaf]) {
+// points 4g..4g+3 (vector loads in the integrand).
+template <typename S, int NT>
+__device__ __forceinline__ void grad_item(const BuildArgs &a, const S *__restrict__ ao,
+                                          const double *__restrict__ ao2,
+                                          const int *__restrict__ ao_map, const DenItem &it,
+                                          double *__restrict__ gpart, char *s_stage) {
+  using P = GradDma<S, NT>;
+  constexpr int CT = NT == 4 ? 2 : 4;  // column tiles of a wavefront
+  const LeafDev L = a.leaves[it.leaf];
+  double *gp = gpart + 3LL * (L.map_off + it.c0);
+  const int t = threadIdx.x, lane = t & 63;
+  if (!a.leaf_active[it.leaf]) {
     // skipped by the max-rho rule (dft_gradient_kernels.cpp:488-491)
-    for (int i = threadIdx.x; i < 3 * L.mp; i += blockDim.x) gp[i] = 0.0;
+    for (int i = t; i < 3 * it.wc; i += 256) gp[i] = 0.0;
     return;
   }
-  constexpr int NC = GGA ? 4 : 1;
-  for (int i = threadIdx.x; i < L.np; i += blockDim.x)
-#pragma unroll
-    for (int q = 0; q < NC; ++q) s_c[q][i] = a.coef[q * a.ptot + L.pt_off + i];
-  __syncthreads();
   const MolDev MD = a.mols[L.mol];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int l16 = lane & 15, g = lane >> 4;
+  const int wp = wave & 1, wc = wave >> 1;
+  const int hc = it.wc >> 1;
   const int pa = 4 * (l16 & 3) + (l16 >> 2);
   const long long cs = (long long)L.mp * L.np;
   const S *phi = ao + L.ao_off;
   // gradient of phi: cache components 1..3 (GGA) or the extra block (LDA);
   // Hessian xx,xy,xz,yy,yz,zz: the extra block (GGA)
-  const double *x2 = ao2 + L.ao_off / a.ncomp * (GGA ? 6 : 3);
+  const double *x2 = ao2 + L.ao_off / a.ncomp * (NT == 1 ? 3 : 6);
   const double *Dm = a.D2 + MD.moff;
-  const int *map = a.ao_map + L.map_off;
-  for (int c = 32 * wave; c < L.mp; c += 128) {
-    const int gn0 = map[c + l16], gn1 = map[c + 16 + l16];
-    double gs[2][3];
+  const int *map = ao_map + L.map_off;
+  // addresses are a wavefront-uniform base plus a 32-bit lane offset in bytes
+  // (at most a leaf's plane, 16 MB): 64-bit ones per load fill the registers
+  unsigned colbase[P::CW / 32];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) gs[j][0] = gs[j][1] = gs[j][2] = 0.0;
-    for (int p0 = 0; p0 < L.np; p0 += 32) {
-      d4 accT[2][2], accU[2][2];
+  for (int cb = 0; cb < P::CW / 32; ++cb)
+    colbase[cb] = 8u * map[it.c0 + min(32 * cb + (lane >> 1), it.wc - 1)] + 4u * (lane & 1);
+  // plane rows: LPR lanes a row of 64 points, RPI rows a load
+  constexpr int LPR = kGp * (int)sizeof(S) / 16, RPI = 64 / LPR;
+  const int q0 = P::NQ == 4 ? wave : 0;
+  const S *src = phi + q0 * cs;
+  const unsigned loff = (unsigned)((lane / LPR) * L.np) * (unsigned)sizeof(S) + 16u * (lane % LPR);
+  auto dma = [&](int p0, int k0, char *st) __attribute__((always_inline)) {
+    long long kmap[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int r = 0; r < 2; ++r) kmap[r] = (long long)map[k0 + 2 * wave + r] * MD.nbf;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) accT[i][j] = accU[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      double ca[2][4];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) ca[i][q] = (GGA || q == 0) ? s_c[q][p0 + 16 * i + pa] : 0.0;
-      for (int mc = 0; mc < L.mp; mc += 16) {
-#pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const int mu = mc + 4 * g + s4;
-          const long long ro = (long long)mu * L.np + p0 + pa;
-          const long long col = (long long)map[mu] * MD.nbf;
-          const double f0 = (double)phi[ro], f1 = (double)phi[ro + 16];
-          const double d0 = Dm[col + gn0], d1 = Dm[col + gn1];
-          accT[0][0] = mma(f0, d0, accT[0][0]);
-          accT[0][1] = mma(f0, d1, accT[0][1]);
-          accT[1][0] = mma(f1, d0, accT[1][0]);
-          accT[1][1] = mma(f1, d1, accT[1][1]);
-          if (GGA) {
-            const double u0 = ca[0][0] * f0 + ca[0][1] * (double)phi[cs + ro] +
-                              ca[0][2] * (double)phi[2 * cs + ro] +
-                              ca[0][3] * (double)phi[3 * cs + ro];
-            const double u1 = ca[1][0] * f1 + ca[1][1] * (double)phi[cs + ro + 16] +
-                              ca[1][2] * (double)phi[2 * cs + ro + 16] +
-                              ca[1][3] * (double)phi[3 * cs + ro + 16];
-            accU[0][0] = mma(u0, d0, accU[0][0]);
-            accU[0][1] = mma(u0, d1, accU[0][1]);
-            accU[1][0] = mma(u1, d0, accU[1][0]);
-            accU[1][1] = mma(u1, d1, accU[1][1]);
-          }
-        }
-      }
-      // integrand at the lane's 4 points of each tile for its AO column
-#pragma unroll
-      for (int pt = 0; pt < 2; ++pt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          const int pb = p0 + pt * 16 + 4 * g;
-          const long long off = (long long)(c + nt * 16 + l16) * L.np + pb;
-          d4 gx, gy, gz;
-          if (GGA) {
-            gx = load4d<S>(phi + cs + off);
-            gy = load4d<S>(phi + 2 * cs + off);
-            gz = load4d<S>(phi + 3 * cs + off);
-          } else {
-            gx = load4d<double>(x2 + off);
-            gy = load4d<double>(x2 + cs + off);
-            gz = load4d<double>(x2 + 2 * cs + off);
-          }
-          if (!GGA) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const double t = 2.0 * s_c[0][pb + r] * accT[pt][nt][r];
-              gs[nt][0] += gx[r] * t;
-              gs[nt][1] += gy[r] * t;
-              gs[nt][2] += gz[r] * t;
-            }
-          } else {
-            const d4 hxx = load4d<double>(x2 + off), hxy = load4d<double>(x2 + cs + off),
-                     hxz = load4d<double>(x2 + 2 * cs + off),
-                     hyy = load4d<double>(x2 + 3 * cs + off),
-                     hyz = load4d<double>(x2 + 4 * cs + off),
-                     hzz = load4d<double>(x2 + 5 * cs + off);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const double c0 = s_c[0][pb + r], c1 = s_c[1][pb + r], c2 = s_c[2][pb + r],
-                           c3 = s_c[3][pb + r];
-              const double t = accT[pt][nt][r], u = accU[pt][nt][r];
-              gs[nt][0] += gx[r] * u + (c0 * gx[r] + c1 * hxx[r] + c2 * hxy[r] + c3 * hxz[r]) * t;
-              gs[nt][1] += gy[r] * u + (c0 * gy[r] + c1 * hxy[r] + c2 * hyy[r] + c3 * hyz[r]) * t;
-              gs[nt][2] += gz[r] * u + (c0 * gz[r] + c1 * hxz[r] + c2 * hyz[r] + c3 * hzz[r]) * t;
-            }
-          }
-        }
+    for (int i = 0; i < P::PL; ++i) {
+      // LDA: the plane's loads shared out over the wavefronts (with FP32
+      // storage wavefronts w and w + 2 load the same rows)
+      const int ii = P::NQ == 4 ? i : (wave + 4 * i) % P::PI;
+      __builtin_amdgcn_global_load_lds(at(src + (long long)(k0 + ii * RPI) * L.np + p0, loff),
+                                       st + q0 * P::PLANE + ii * 1024, 16, 0, 0);
     }
-    // sum over the four lane groups (the points) of each AO column
+    char *sd = st + P::NQ * P::PLANE;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double v = gs[nt][k];
-        v += __shfl_xor(v, 16, 64);
-        v += __shfl_xor(v, 32, 64);
-        if (g == 0) gp[3 * (c + nt * 16 + l16) + k] = v;
+      for (int cb = 0; cb < P::CW / 32; ++cb)
+        __builtin_amdgcn_global_load_lds(at(Dm + kmap[r], colbase[cb]),
+                                         sd + ((2 * wave + r) * P::CW + 32 * cb) * 8, 4, 0, 0);
+  };
+  double(*s_c)[kGp] = reinterpret_cast<double(*)[kGp]>(s_stage + P::NS * P::STAGE);
+  const int nch = (L.m + kGk - 1) / kGk;
+  const int CTl = live_tiles(L.m - (it.c0 + wc * hc), hc);
+  double gs[CT][3];
+#pragma unroll
+  for (int j = 0; j < CT; ++j) gs[j][0] = gs[j][1] = gs[j][2] = 0.0;
+  auto body = [&](auto Cn) __attribute__((always_inline)) {
+    constexpr int NCt = decltype(Cn)::value;
+    for (int p0 = 0; p0 < L.n; p0 += kGp) {
+      __syncthreads();  // the previous points' buffers and coefficients are consumed
+      for (int c = 0; c < P::NS - 1 && c < nch; ++c) dma(p0, c * kGk, s_stage + c * P::STAGE);
+      for (int i = t; i < P::NC * kGp; i += 256) {
+        const int q = i / kGp, p = i % kGp;
+        s_c[q][p] = q == 4 ? 2.0 * a.coef_tau[L.pt_off + p0 + p] : a.coef[q * a.ptot + L.pt_off + p0 + p];
       }
-  }
-}
-
-// Meta-GGA tau terms (accumulate_gradient_contribution_R<2>,
-// dft_gradient_kernels.cpp:152-172): V_k += sum_j d_kj phi^T ((vtau / 2) d_j phi)
-// contracted with P, i.e. per AO mu and direction k
-//   sum_p sum_j d_kj phi_mu (vtau / 2) T_j,mu,   T_j = (d_j Phi) P,
-// with vtau / 2 = 2 c_tau (c_tau = w vtau / 4, a.coef_tau), into gpart in the
-// normalisation of k_xc_grad's partials.  Same leaf / chunk / point-block
-// structure as k_xc_grad: the three T_j of a chunk and point block on the
-// FP64 matrix cores (A operand d_j phi from the AO cache, B operand P
-// gathered through the AO map), the Hessian from ao2 in the integrand.
-template <typename S>
-__global__ __launch_bounds__(256, 2) void k_xc_grad_tau(BuildArgs a, const S *__restrict__ ao,
-                                                       const double *__restrict__ ao2,
-                                                       double *__restrict__ gpart) {
-  __shared__ double s_t[kMaxLeafPts];
-  const int leaf = xcd_leaf(blockIdx.x, gridDim.x);
-  const LeafDev L = a.leaves[leaf];
-  double *gp = gpart + 3LL * L.map_off;
-  if (!a.leaf_active[leaf]) {
-    for (int i = threadIdx.x; i < 3 * L.mp; i += blockDim.x) gp[i] = 0.0;
-    return;
-  }
-  for (int i = threadIdx.x; i < L.np; i += blockDim.x)
-    s_t[i] = 2.0 * a.coef_tau[L.pt_off + i];
-  __syncthreads();
-  const MolDev MD = a.mols[L.mol];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int l16 = lane & 15, g = lane >> 4;
-  const int pa = 4 * (l16 & 3) + (l16 >> 2);
-  const long long cs = (long long)L.mp * L.np;
-  const S *phi = ao + L.ao_off;
-  const double *x2 = ao2 + L.ao_off / a.ncomp * 6;
-  const double *Dm = a.D2 + MD.moff;
-  const int *map = a.ao_map + L.map_off;
-  for (int c = 32 * wave; c < L.mp; c += 128) {
-    const int gn0 = map[c + l16], gn1 = map[c + 16 + l16];
-    double gs[2][3];
+      d4 acc[NT][2][CT];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) gs[j][0] = gs[j][1] = gs[j][2] = 0.0;
-    for (int p0 = 0; p0 < L.np; p0 += 32) {
-      d4 acc[3][2][2];
-#pragma unroll
-      for (int d = 0; d < 3; ++d)
+      for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[d][i][j] = d4{0.0, 0.0, 0.0, 0.0};
-      for (int mc = 0; mc < L.mp; mc += 16) {
+          for (int j = 0; j < CT; ++j) acc[n][i][j] = d4{0.0, 0.0, 0.0, 0.0};
+      const bool any = L.n > p0 + 32 * wp;  // the wavefront's points hold real ones
+      double ca[2][4];
+      int cur = 0;
+      for (int c = 0; c < nch; ++c) {
+        if (c + 1 < nch && c > 0) vmcnt_barrier<P::LOADS>();
+        else vmcnt_barrier<0>();  // the first also waits for the coefficients
+        if (NT == 2 && c == 0) {
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-          const int mu = mc + 4 * g + s4;
-          const long long ro = (long long)mu * L.np + p0 + pa;
-          const long long col = (long long)map[mu] * MD.nbf;
-          const double d0 = Dm[col + gn0], d1 = Dm[col + gn1];
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const double f0 = (double)phi[(d + 1) * cs + ro];
-            const double f1 = (double)phi[(d + 1) * cs + ro + 16];
-            acc[d][0][0] = mma(f0, d0, acc[d][0][0]);
-            acc[d][0][1] = mma(f0, d1, acc[d][0][1]);
-            acc[d][1][0] = mma(f1, d0, acc[d][1][0]);
-            acc[d][1][1] = mma(f1, d1, acc[d][1][1]);
+            for (int q = 0; q < 4; ++q) ca[i][q] = s_c[q][32 * wp + 16 * i + pa];
+        }
+        const int nxt = cur == 0 ? P::NS - 1 : cur - 1;
+        if (c + P::NS - 1 < nch) dma(p0, (c + P::NS - 1) * kGk, s_stage + nxt * P::STAGE);
+        const S *sp = reinterpret_cast<const S *>(s_stage + cur * P::STAGE);
+        const double *sd = reinterpret_cast<const double *>(s_stage + cur * P::STAGE + P::NQ * P::PLANE);
+        if (NCt > 0 && any) {
+#pragma unroll
+          for (int ks = 0; ks < kGk / 4; ++ks) {
+            const int kk = 4 * ks + g;
+            double yv[NCt ? NCt : 1], xv[P::NQ][2];
+#pragma unroll
+            for (int j = 0; j < NCt; ++j) yv[j] = sd[kk * P::CW + wc * hc + 16 * j + l16];
+#pragma unroll
+            for (int q = 0; q < P::NQ; ++q)
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                xv[q][i] = (double)sp[(q * kGk + kk) * kGp + 32 * wp + 16 * i + pa];
+            if constexpr (NT == 2) {
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                xv[1][i] = ca[i][0] * xv[0][i] + ca[i][1] * xv[1][i] + ca[i][2] * xv[2][i] +
+                           ca[i][3] * xv[3][i];
+            }
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < NCt; ++j) acc[n][i][j] = mma(xv[n][i], yv[j], acc[n][i][j]);
+          }
+        }
+        cur = cur + 1 == P::NS ? 0 : cur + 1;
+      }
+      // the integrand at the lane's 4 points of each tile for its AO column
+      if (!any) continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int j = 0; j < NCt; ++j) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            // two points of a tile at a time; an opaque 0 (no instruction) and
+            // a scheduling barrier keep each round's addresses, loads and
+            // coefficients in the round: shared between rounds they spill
+            int zero = 0;
+            asm volatile("" : "+s"(zero));
+            __builtin_amdgcn_sched_barrier(0);
+            const int pl = 32 * wp + 16 * i + 4 * g + 2 * h + zero;
+            const unsigned off = (unsigned)((it.c0 + wc * hc + 16 * j + l16) * L.np + p0 + pl);
+            auto hess = [&](int k) __attribute__((always_inline)) {
+              return load2d<double>(at(x2 + k * cs, 8u * off));
+            };
+            auto grad = [&](int k) __attribute__((always_inline)) {
+              return load2d<S>(at(phi + k * cs, (unsigned)sizeof(S) * off));
+            };
+            if constexpr (NT == 1) {
+              const d2 gx = hess(0), gy = hess(1), gz = hess(2);  // the gradient planes
+#pragma unroll
+              for (int r = 0; r < 2; ++r) {
+                const double v = 2.0 * s_c[0][pl + r] * acc[0][i][j][2 * h + r];
+                gs[j][0] += gx[r] * v;
+                gs[j][1] += gy[r] * v;
+                gs[j][2] += gz[r] * v;
+              }
+            } else {
+              const d2 gx = grad(1), gy = grad(2), gz = grad(3);
+              const d2 hxx = hess(0), hxy = hess(1), hxz = hess(2), hyy = hess(3), hyz = hess(4),
+                       hzz = hess(5);
+#pragma unroll
+              for (int r = 0; r < 2; ++r) {
+                const double c0 = s_c[0][pl + r], c1 = s_c[1][pl + r], c2 = s_c[2][pl + r],
+                             c3 = s_c[3][pl + r];
+                const double v = acc[0][i][j][2 * h + r];
+                double u, b1 = c1 * v, b2 = c2 * v, b3 = c3 * v;
+                if constexpr (NT == 2) {
+                  u = acc[1][i][j][2 * h + r] + c0 * v;
+                } else {
+                  const double ct = s_c[P::NC - 1][pl + r];
+                  const double tx = acc[1][i][j][2 * h + r], ty = acc[2][i][j][2 * h + r],
+                               tz = acc[3][i][j][2 * h + r];
+                  u = 2.0 * c0 * v + c1 * tx + c2 * ty + c3 * tz;
+                  b1 += ct * tx;
+                  b2 += ct * ty;
+                  b3 += ct * tz;
+                }
+                gs[j][0] += gx[r] * u + (b1 * hxx[r] + b2 * hxy[r] + b3 * hxz[r]);
+                gs[j][1] += gy[r] * u + (b1 * hxy[r] + b2 * hyy[r] + b3 * hyz[r]);
+                gs[j][2] += gz[r] * u + (b1 * hxz[r] + b2 * hyz[r] + b3 * hzz[r]);
+              }
+            }
           }
         }
       }
-#pragma unroll
-      for (int pt = 0; pt < 2; ++pt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          const int pb = p0 + pt * 16 + 4 * g;
-          const long long off = (long long)(c + nt * 16 + l16) * L.np + pb;
-          const d4 hxx = load4d<double>(x2 + off), hxy = load4d<double>(x2 + cs + off),
-                   hxz = load4d<double>(x2 + 2 * cs + off),
-                   hyy = load4d<double>(x2 + 3 * cs + off),
-                   hyz = load4d<double>(x2 + 4 * cs + off),
-                   hzz = load4d<double>(x2 + 5 * cs + off);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const double ct = s_t[pb + r];
-            const double tx = ct * acc[0][pt][nt][r], ty = ct * acc[1][pt][nt][r],
-                         tz = ct * acc[2][pt][nt][r];
-            gs[nt][0] += hxx[r] * tx + hxy[r] * ty + hxz[r] * tz;
-            gs[nt][1] += hxy[r] * tx + hyy[r] * ty + hyz[r] * tz;
-            gs[nt][2] += hxz[r] * tx + hyz[r] * ty + hzz[r] * tz;
-          }
-        }
     }
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double v = gs[nt][k];
-        v += __shfl_xor(v, 16, 64);
-        v += __shfl_xor(v, 32, 64);
-        if (g == 0) gp[3 * (c + nt * 16 + l16) + k] = v;
-      }
+  };
+  switch (CTl) {
+  case 0: body(std::integral_constant<int, 0>{}); break;
+  case 2: body(std::integral_constant<int, 2>{}); break;
+  case 3: body(std::integral_constant<int, CT < 3 ? CT : 3>{}); break;
+  default: body(std::integral_constant<int, CT>{}); break;
   }
+  // sums over the four lane groups, then over the two wavefronts of a column half
+  double *s_g = reinterpret_cast<double *>(s_stage);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < CT; ++j)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      double v = gs[j][k];
+      v += __shfl_xor(v, 16, 64);
+      v += __shfl_xor(v, 32, 64);
+      gs[j][k] = v;
+      if (wp == 1 && g == 0) s_g[3 * (64 * wc + 16 * j + l16) + k] = v;
+    }
+  __syncthreads();
+  if (wp == 0 && g == 0)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      if (16 * j >= hc) break;
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        gp[3 * (wc * hc + 16 * j + l16) + k] = gs[j][k] + s_g[3 * (64 * wc + 16 * j + l16) + k];
+    }
 }
 
-// grad[3 A + k] = -2 sum of gpart (plus gpart2, the beta spin of an
-// unrestricted gradient, when given) over the entries of atom A, in a fixed
-// order (per-thread strided sums, then a fixed tree).
+template <typename S, int NT>
+__global__ __launch_bounds__(256, 2) void k_xc_grad(BuildArgs a, const S *__restrict__ ao,
+                                                   const double *__restrict__ ao2,
+                                                   const int *__restrict__ ao_map,
+                                                   const DenItem *__restrict__ items,
+                                                   double *__restrict__ gpart) {
+  using P = GradDma<S, NT>;
+  __shared__ __align__(16) char s_stage[P::NS * P::STAGE + P::NC * kGp * 8];
+  static_assert(P::STAGE >= 3 * 128 * 8, "the column sums fit");
+  const DenItem it = items[blockIdx.x];
+  if (it.leaf < 0) return;
+  grad_item<S, NT>(a, ao, ao2, ao_map, it, gpart, s_stage);
+}
+
+// Per-atom sums in a fixed order: block (A, y) sums every kGradSplit-th run of
+// 256 entries of atom A (per-thread strided sums, then a fixed tree), then
+// grad[3 A + k] = -2 times the sum of the atom's blocks.  gpart2: the beta spin
+// of an unrestricted gradient (null otherwise).  With one block per atom a
+// 96-atom cluster's 2e6 entries kept 96 of the 256 CUs busy for 134 us.
 __global__ __launch_bounds__(256) void k_grad_reduce(const double *__restrict__ gpart,
                                                      const double *__restrict__ gpart2,
-                                                     const double *__restrict__ gpart3,
-                                                     const double *__restrict__ gpart4,
                                                      const int *__restrict__ atom_off,
                                                      const int *__restrict__ atom_ent,
-                                                     double *__restrict__ grad) {
+                                                     double *__restrict__ red) {
   __shared__ double s_r[3][256];
   const int A = blockIdx.x;
   const int e0 = atom_off[A], e1 = atom_off[A + 1];
   double v[3] = {0.0, 0.0, 0.0};
-  for (int i = e0 + threadIdx.x; i < e1; i += blockDim.x) {
+  for (int i = e0 + blockIdx.y * 256 + threadIdx.x; i < e1; i += 256 * kGradSplit) {
     const long long e = 3LL * atom_ent[i];
     v[0] += gpart[e];
     v[1] += gpart[e + 1];
@@ -307,11 +342,6 @@ __global__ __launch_bounds__(256) void k_grad_reduce(const double *__restrict__ 
       v[0] += gpart2[e];
       v[1] += gpart2[e + 1];
       v[2] += gpart2[e + 2];
-    }
-    if (gpart3) {
-      v[0] += gpart3[e] + gpart4[e];
-      v[1] += gpart3[e + 1] + gpart4[e + 1];
-      v[2] += gpart3[e + 2] + gpart4[e + 2];
     }
   }
 #pragma unroll
@@ -323,7 +353,15 @@ __global__ __launch_bounds__(256) void k_grad_reduce(const double *__restrict__ 
       for (int k = 0; k < 3; ++k) s_r[k][threadIdx.x] += s_r[k][threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x < 3) grad[3 * A + threadIdx.x] = -2.0 * s_r[threadIdx.x][0];
+  if (threadIdx.x < 3) red[(A * kGradSplit + blockIdx.y) * 3 + threadIdx.x] = s_r[threadIdx.x][0];
+}
+
+__global__ void k_grad_final(const double *__restrict__ red, int n3, double *__restrict__ grad) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n3) return;
+  double v = 0.0;
+  for (int y = 0; y < kGradSplit; ++y) v += red[(i / 3 * kGradSplit + y) * 3 + i % 3];
+  grad[i] = -2.0 * v;
 }
 
 void check(const char *what) {
@@ -334,57 +372,26 @@ void check(const char *what) {
 } // namespace
 
 void launch_xc_gradient_partials(const BuildArgs &a, const void *ao, bool ao_fp32,
-                                 const double *ao2, double *gpart, hipStream_t s) {
-  if (a.nleaves == 0) return;
-  const bool gga = a.deriv != 0;
-  if (ao_fp32) {
-    const float *p = static_cast<const float *>(ao);
-    if (gga) k_xc_grad<float, true><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-    else k_xc_grad<float, false><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-  } else {
-    const double *p = static_cast<const double *>(ao);
-    if (gga) k_xc_grad<double, true><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-    else k_xc_grad<double, false><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-  }
+                                 const double *ao2, const DenItem *items, int nitems,
+                                 double *gpart, hipStream_t s) {
+  if (a.nleaves == 0 || nitems == 0) return;
+  auto launch = [&](auto s_tag) {
+    using S = decltype(s_tag);
+    (a.deriv == 0 ? k_xc_grad<S, 1> : a.coef_tau ? k_xc_grad<S, 4> : k_xc_grad<S, 2>)
+        <<<nitems, 256, 0, s>>>(a, static_cast<const S *>(ao), ao2, a.ao_map, items, gpart);
+  };
+  if (ao_fp32) launch(float{});
+  else launch(double{});
   check("k_xc_grad");
 }
 
-void launch_xc_gradient_tau(const BuildArgs &a, const void *ao, bool ao_fp32,
-                            const double *ao2, double *gpart, hipStream_t s) {
-  if (a.nleaves == 0) return;
-  if (ao_fp32)
-    k_xc_grad_tau<float><<<a.nleaves, 256, 0, s>>>(a, static_cast<const float *>(ao), ao2, gpart);
-  else
-    k_xc_grad_tau<double><<<a.nleaves, 256, 0, s>>>(a, static_cast<const double *>(ao), ao2, gpart);
-  check("k_xc_grad_tau");
-}
-
 void launch_grad_reduce(const double *gpart, const double *gpart2, int natoms,
-                        const int *atom_off, const int *atom_ent, double *grad, hipStream_t s,
-                        const double *gpart3, const double *gpart4) {
-  k_grad_reduce<<<natoms, 256, 0, s>>>(gpart, gpart2, gpart3, gpart4, atom_off, atom_ent, grad);
+                        const int *atom_off, const int *atom_ent, double *red, double *grad,
+                        hipStream_t s) {
+  k_grad_reduce<<<dim3(natoms, kGradSplit), 256, 0, s>>>(gpart, gpart2, atom_off, atom_ent, red);
   check("k_grad_reduce");
-}
-
-void launch_xc_gradient(const BuildArgs &a, const void *ao, bool ao_fp32, const double *ao2,
-                        double *gpart, int natoms, const int *atom_off, const int *atom_ent,
-                        double *grad, hipStream_t s) {
-  if (a.nleaves > 0) {
-    const bool gga = a.deriv != 0;
-    if (ao_fp32) {
-      const float *p = static_cast<const float *>(ao);
-      if (gga) k_xc_grad<float, true><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-      else k_xc_grad<float, false><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-    } else {
-      const double *p = static_cast<const double *>(ao);
-      if (gga) k_xc_grad<double, true><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-      else k_xc_grad<double, false><<<a.nleaves, 256, 0, s>>>(a, p, ao2, gpart);
-    }
-    check("k_xc_grad");
-  }
-  k_grad_reduce<<<natoms, 256, 0, s>>>(gpart, nullptr, nullptr, nullptr, atom_off, atom_ent,
-                                       grad);
-  check("k_grad_reduce");
+  k_grad_final<<<(3 * natoms + 255) / 256, 256, 0, s>>>(red, 3 * natoms, grad);
+  check("k_grad_final");
 }
 
 } // namespace occxc

@@ -223,24 +223,21 @@ void launch_ao_residuals(const BuildArgs &a, const void *ao, hipStream_t s);
 void launch_ao_extra(const BuildArgs &a, double *out, bool hessian, hipStream_t s);
 // XC gradient contraction (grad.hip): per leaf and local AO mu the sum over
 // the leaf's points of the gradient integrand into gpart[3 (map_off + mu) + k],
-// then grad[3 A + k] = -2 sum over the entries of atom A (CSR atom_off /
-// atom_ent), in a fixed order.
-// the same in two steps: per-AO partials of one spin density (a.D2 and
-// a.coef of that spin), then the per-atom reduction of one or two partial sets
+// for one spin density (a.D2 and a.coef of that spin; a.coef_tau adds the
+// meta-GGA's tau terms).  items: a leaf and one of its column blocks each, at
+// most kGradWide AOs wide (kGradWideTau with a.coef_tau); leaf < 0 is padding.
+constexpr int kGradPoints = 64;  // points a gradient item takes at a time
+constexpr int kGradWide = 128, kGradWideTau = 64;
 void launch_xc_gradient_partials(const BuildArgs &a, const void *ao, bool ao_fp32,
-                                 const double *ao2, double *gpart, hipStream_t s);
-// restricted meta-GGA: the tau terms' per-AO partials (a.coef_tau, Hessian in
-// ao2) into gpart, reduced together with k_xc_grad's by launch_grad_reduce
-void launch_xc_gradient_tau(const BuildArgs &a, const void *ao, bool ao_fp32,
-                            const double *ao2, double *gpart, hipStream_t s);
-// grad = -2 sum of up to four partial sets (gpart2, gpart3/gpart4 optional;
-// gpart3 and gpart4 come together)
+                                 const double *ao2, const DenItem *items, int nitems,
+                                 double *gpart, hipStream_t s);
+// grad[3 A + k] = -2 sum of the partials (of both spins when gpart2 is given)
+// over the entries of atom A (CSR atom_off / atom_ent), in a fixed order; red
+// holds 3 kGradSplit natoms doubles
+constexpr int kGradSplit = 16;
 void launch_grad_reduce(const double *gpart, const double *gpart2, int natoms,
-                        const int *atom_off, const int *atom_ent, double *grad, hipStream_t s,
-                        const double *gpart3 = nullptr, const double *gpart4 = nullptr);
-void launch_xc_gradient(const BuildArgs &a, const void *ao, bool ao_fp32, const double *ao2,
-                        double *gpart, int natoms, const int *atom_off, const int *atom_ent,
-                        double *grad, hipStream_t s);
+                        const int *atom_off, const int *atom_ent, double *red, double *grad,
+                        hipStream_t s);
 void launch_density_functional(const BuildArgs &a, const void *ao, bool fp32,
                                hipStream_t s);
 void launch_vxc(const BuildArgs &a, const void *ao, bool fp32, hipStream_t s);

@@ -75,3 +75,26 @@ def test_unrestricted_build_matches_oracle(system, basis_name, tile, method, pre
     assert abs(e - exc) <= (1e-11 if precision == "fp64" else 1e-6)
     assert np.abs(np.array(n) - np.array(nel)).max() <= (1e-11 if precision == "fp64" else 1e-6)
     ctx.close()
+
+
+# gradients: sums over the leaf points of values up to ~1e2 (core derivatives),
+# rounded at 1e-15 of them: 1e-11; FP32 storage 6e-8 of an entry, 1e-6 in all
+@pytest.mark.parametrize("precision", ["fp64", "fp32cache"])
+@pytest.mark.parametrize("method", ["svwn5", "pbe", "tpss"])
+@pytest.mark.parametrize("system,basis_name", [
+    ("water", "6-31g"), ("methane", "def2-svp"), ("water3", "def2-tzvp"), ("alkane5", "6-31g")])
+def test_gradients_match_oracle(system, basis_name, method, precision):
+    basis, pts, wts, ctx = _setup(system, basis_name, method, precision, 0)
+    ob, n = oracle.OracleBasis.from_flat(basis.flat()), len(basis.atoms)
+    tol = 1e-11 if precision == "fp64" else 1e-6
+    D = random_density(basis.nbf, 5, 31)
+    G = oracle.xc_gradient(ob, basis.shell_atom, n, pts, wts, functional_ids(method), D)
+    first = ctx.xc_gradient(D, basis.shell_atom, n)
+    assert np.abs(first - G).max() <= tol * max(1.0, np.abs(G).max())
+    assert np.array_equal(first, ctx.xc_gradient(D, basis.shell_atom, n))
+    Du = np.asfortranarray(np.concatenate([D, random_density(basis.nbf, 4, 32)]) / 2)
+    Gu = oracle.xc_gradient_unrestricted(ob, basis.shell_atom, n, pts, wts,
+                                         functional_ids(method), Du)
+    got = ctx.xc_gradient_unrestricted(Du, basis.shell_atom, n)
+    assert np.abs(got - Gu).max() <= tol * max(1.0, np.abs(Gu).max())
+    ctx.close()
