@@ -13,13 +13,13 @@
 //
 // Layout: the context's points are in leaf order; k_vv10_prep scatters each
 // real point's (x, y, z, rho w, omega0, kappa, rho) into input-order planes
-// of npts; k_vv10_pairs gives F, U, W per input point (one thread per i,
-// 256-point j tiles in LDS, blocks with the most j tiles first);
-// k_vv10_coef gathers them back per leaf and forms the weighted
+// of npts; k_vv10_pairs gives partial sums of F, U, W per input point and
+// segment of j; k_vv10_coef adds them up per leaf point and forms the weighted
 // exc / vrho / vsigma and the GGA Vxc coefficients, which the restricted Vxc
 // kernel contracts (Vxc = ktmp + ktmp^T, nonlocal_correlation.cpp:295-303).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <stdexcept>
 #include <string>
@@ -31,9 +31,26 @@ namespace {
 
 constexpr double kVvPi = 3.14159265358979323846;
 constexpr double kVvRhoMin = 1e-8;  // nonlocal_correlation.cpp:68,77
-constexpr int kVvTile = 256;
+constexpr int kVvTile = 256;   // j points of a tile
+constexpr int kVvRows = 512;   // i points of a block, two per thread
+constexpr int kVvSegs = 16;    // most segments of j
 
-enum : int { kX = 0, kY, kZ, kRW, kOM, kKA, kRHO, kF, kU, kW, kNlcPlanes };
+enum : int { kX = 0, kY, kZ, kRW, kOM, kKA, kRHO, kNlcPlanes };
+
+// Segments of j: runs of `tiles` tiles, so that the triangle of pairs becomes
+// many units of about equal work (one workgroup per 256 points with all of its
+// j tiles left a quarter of the chip idle at the end: 1032 workgroups, all
+// resident at once, the longest twice the average).
+struct VvSegs {
+  int tiles, n;
+};
+VvSegs vv_segs(long long npts) {
+  const long long nt = (npts + kVvTile - 1) / kVvTile;
+  VvSegs g;
+  g.tiles = (int)std::max<long long>(8, (nt + kVvSegs - 1) / kVvSegs);
+  g.n = (int)std::max<long long>(1, (nt + g.tiles - 1) / g.tiles);
+  return g;
+}
 
 void check(const char *what) {
   const hipError_t e = hipGetLastError();
@@ -97,7 +114,7 @@ __global__ __launch_bounds__(256) void k_vv10_prep(BuildArgs a, const double *__
 
 // 1/x for the pair denominators: the hardware reciprocal refined by two
 // Newton-Raphson steps, r <- r + r (1 - x r) (within about an ulp; x lies in
-// [1e-3, 1e30] here: g >= kappa(1e-8) ~ 0.7, so no scaling is needed)
+// [1e-3, 1e30] in ordinary use: g >= kappa(1e-8) ~ 0.7, so no scaling is needed)
 __device__ inline double recip(double x) {
   double r = __builtin_amdgcn_rcp(x);
   r = fma(r, fma(-x, r, 1.0), r);
@@ -105,63 +122,152 @@ __device__ inline double recip(double x) {
   return r;
 }
 
-// F, U, W of every input point i from the points j < i.  Block b (heaviest
-// first) owns points [256 b, 256 b + 256) and walks the j tiles 0..b; dead j
-// (rho_j < 1e-8, or beyond npts) enter with weight 0, which adds exactly 0.
-// One reciprocal per pair: R = 1 / ((g_i s)^2 g_j), s = g_i + g_j, gives
-// t = 2 rho_j w_j / (g_i g_j s) = q (g_i s) R and t (1/g_i + 1/s) = q (s + g_i) R.
-// The loop is FP64 VALU-bound (about 24 instructions per pair).
-__global__ __launch_bounds__(256) void k_vv10_pairs(double *__restrict__ nlc, long long npts) {
-  __shared__ double s_x[kVvTile], s_y[kVvTile], s_z[kVvTile], s_q[kVvTile], s_om[kVvTile],
-      s_ka[kVvTile];
-  const long long blk = (long long)gridDim.x - 1 - blockIdx.x;
-  const long long i = blk * kVvTile + threadIdx.x;
-  const bool in = i < npts;
-  const bool live = in && nlc[kRHO * npts + i] >= kVvRhoMin;
-  double xi = 0, yi = 0, zi = 0, omi = 0, kai = 1, f = 0, u = 0, w = 0;
-  if (live) {
-    xi = nlc[kX * npts + i];
-    yi = nlc[kY * npts + i];
-    zi = nlc[kZ * npts + i];
-    omi = nlc[kOM * npts + i];
-    kai = nlc[kKA * npts + i];
-    f = nlc[kRW * npts + i] / (2 * kai * kai * kai);
-    u = f * (1.0 / kai + 1.0 / (2 * kai));
-  }
-  for (long long j0 = 0; j0 <= blk * kVvTile; j0 += kVvTile) {
-    __syncthreads();
-    const long long j = j0 + threadIdx.x;
-    const bool lj = j < npts && nlc[kRHO * npts + j] >= kVvRhoMin;
-    s_x[threadIdx.x] = lj ? nlc[kX * npts + j] : 0.0;
-    s_y[threadIdx.x] = lj ? nlc[kY * npts + j] : 0.0;
-    s_z[threadIdx.x] = lj ? nlc[kZ * npts + j] : 0.0;
-    s_q[threadIdx.x] = lj ? 2.0 * nlc[kRW * npts + j] : 0.0;
-    s_om[threadIdx.x] = lj ? nlc[kOM * npts + j] : 0.0;
-    s_ka[threadIdx.x] = lj ? nlc[kKA * npts + j] : 1.0;
-    __syncthreads();
-    if (!live) continue;
-    const long long rem = i - j0;  // >= 0: j0 <= blk * kVvTile <= i
-    const int jn = rem < kVvTile ? (int)rem : kVvTile;
-    for (int jj = 0; jj < jn; ++jj) {
-      const double dx = xi - s_x[jj], dy = yi - s_y[jj], dz = zi - s_z[jj];
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      const double gi = r2 * omi + kai;
-      const double gj = r2 * s_om[jj] + s_ka[jj];
-      const double s = gi + gj;
-      const double gis = gi * s;
-      const double R = recip(gis * gis * gj);
-      const double qr = s_q[jj] * R;
-      f += qr * gis;
-      const double tu = qr * (s + gi);
-      u += tu;
-      w += tu * r2;
+// The same for four numbers with one hardware reciprocal: the product's,
+// refined by one third-order step r <- r + r (e + e^2), e = 1 - x r, times the
+// other three.  The product stays in range for the x of vv10_narrow points (at
+// most 1e56, at least 1e-30 each).
+__device__ inline void recip4(double x0, double x1, double x2, double x3, double (&r)[4]) {
+  const double a = x0 * x1, b = x2 * x3, x = a * b;
+  double q = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, q, 1.0);
+  q = fma(q, fma(e, e, e), q);
+  const double qa = q * b, qb = q * a;
+  r[0] = qa * x1;
+  r[1] = qa * x0;
+  r[2] = qb * x3;
+  r[3] = qb * x2;
+}
+
+// Points whose pair denominators (below) recip4 may take: coordinates within
+// 1e3 Bohr and omega0, kappa at most 1e4 give g <= 1.3e11, and kappa >= 1e-6
+// bounds it below.  Others (far larger systems, a tiny b) take one reciprocal
+// a pair.
+__device__ inline bool vv10_narrow(double x, double y, double z, double om, double ka) {
+  return fabs(x) <= 1e3 && fabs(y) <= 1e3 && fabs(z) <= 1e3 && om <= 1e4 && ka <= 1e4 && ka >= 1e-6;
+}
+
+struct VvPoint {
+  double x, y, z, om, ka, f, u, w;
+};
+
+// One pair's terms up to its reciprocal: R = 1 / ((g_i s)^2 g_j), s = g_i + g_j,
+// gives t = 2 rho_j w_j / (g_i g_j s) = q (g_i s) R and t (1/g_i + 1/s) =
+// q (s + g_i) R.
+struct VvPair {
+  double r2, gis, h, den;
+};
+__device__ inline VvPair vv_pair(const VvPoint &p, const double2 &xy, const double2 &zq,
+                                 const double2 &ok) {
+  const double dx = p.x - xy.x, dy = p.y - xy.y, dz = p.z - zq.x;
+  VvPair v;
+  v.r2 = dx * dx + dy * dy + dz * dz;
+  const double gi = v.r2 * p.om + p.ka, gj = v.r2 * ok.x + ok.y, s = gi + gj;
+  v.gis = gi * s;
+  v.h = s + gi;
+  v.den = v.gis * v.gis * gj;
+  return v;
+}
+__device__ inline void vv_add(VvPoint &p, const VvPair &v, double q, double R) {
+  const double qr = q * R;
+  p.f += qr * v.gis;
+  const double tu = qr * v.h;
+  p.u += tu;
+  p.w += tu * v.r2;
+}
+
+// Partial F, U, W of every input point i over the points j < i of one segment.
+// Block (b, seg), b heaviest first, owns points [512 b, 512 b + 512), two a
+// thread, and walks the segment's j tiles up to its own; a j's data is read
+// from LDS once for two pairs, and two j's four pairs share one reciprocal.
+// Dead j (rho_j < 1e-8, or beyond npts) enter with weight 0, which adds exactly
+// 0; the block's own two tiles run pair by pair and stop at i.  FP64
+// VALU-bound: 23 instruction slots a pair (26 with a reciprocal each, 24.5 with
+// one for two).  (H2O)16 / def2-SVP, 50 x 110 grid, 3.5e10 pairs: 32.4 ms with
+// one workgroup per 256 points and a reciprocal each, 22.0 ms now.
+__global__ __launch_bounds__(256) void k_vv10_pairs(const double *__restrict__ nlc, long long npts,
+                                                    int seg_tiles, double *__restrict__ part) {
+  __shared__ double2 s_xy[kVvTile], s_zq[kVvTile], s_ok[kVvTile];
+  const long long b = (long long)gridDim.x - 1 - blockIdx.x;
+  const int seg = blockIdx.y;
+  const long long jt0 = (long long)seg * seg_tiles;
+  if (jt0 > 2 * b + 1) return;
+  const long long jt1 = min(jt0 + seg_tiles, 2 * b + 2);
+  VvPoint p[2];
+  long long i[2];
+  bool live[2], wide = false;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    i[k] = b * kVvRows + k * kVvTile + threadIdx.x;
+    live[k] = i[k] < npts && nlc[kRHO * npts + i[k]] >= kVvRhoMin;
+    p[k] = VvPoint{0, 0, 0, 0, 1, 0, 0, 0};
+    if (live[k]) {
+      p[k].x = nlc[kX * npts + i[k]];
+      p[k].y = nlc[kY * npts + i[k]];
+      p[k].z = nlc[kZ * npts + i[k]];
+      p[k].om = nlc[kOM * npts + i[k]];
+      p[k].ka = nlc[kKA * npts + i[k]];
+      wide = wide || !vv10_narrow(p[k].x, p[k].y, p[k].z, p[k].om, p[k].ka);
+      if (seg == 0) {
+        p[k].f = nlc[kRW * npts + i[k]] / (2 * p[k].ka * p[k].ka * p[k].ka);
+        p[k].u = p[k].f * (1.0 / p[k].ka + 1.0 / (2 * p[k].ka));
+      }
     }
   }
-  if (in) {
-    nlc[kF * npts + i] = live ? f * -1.5 : 0.0;
-    nlc[kU * npts + i] = live ? u : 0.0;
-    nlc[kW * npts + i] = live ? w : 0.0;
+  const bool any = __syncthreads_or(live[0] || live[1]);
+  const bool wide_i = __syncthreads_or(wide);
+  for (long long jt = jt0; any && jt < jt1; ++jt) {
+    __syncthreads();
+    const long long j = jt * kVvTile + threadIdx.x;
+    const bool lj = j < npts && nlc[kRHO * npts + j] >= kVvRhoMin;
+    double2 xy{0, 0}, zq{0, 0}, ok{0, 1};
+    if (lj) {
+      xy = double2{nlc[kX * npts + j], nlc[kY * npts + j]};
+      zq = double2{nlc[kZ * npts + j], 2.0 * nlc[kRW * npts + j]};
+      ok = double2{nlc[kOM * npts + j], nlc[kKA * npts + j]};
+    }
+    s_xy[threadIdx.x] = xy;
+    s_zq[threadIdx.x] = zq;
+    s_ok[threadIdx.x] = ok;
+    const bool wide_j = __syncthreads_or(lj && !vv10_narrow(xy.x, xy.y, zq.x, ok.x, ok.y));
+    if (!wide_i && !wide_j && jt < 2 * b) {
+#pragma unroll 2
+      for (int jj = 0; jj < kVvTile; jj += 2) {
+        VvPair v[4];
+        double q[2], r[4];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          const double2 a = s_xy[jj + m], c = s_zq[jj + m], d = s_ok[jj + m];
+          q[m] = c.y;
+#pragma unroll
+          for (int k = 0; k < 2; ++k) v[2 * m + k] = vv_pair(p[k], a, c, d);
+        }
+        recip4(v[0].den, v[1].den, v[2].den, v[3].den, r);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+          for (int k = 0; k < 2; ++k) vv_add(p[k], v[2 * m + k], q[m], r[2 * m + k]);
+      }
+      continue;
+    }
+    for (int jj = 0; jj < kVvTile; ++jj) {
+      const double2 a = s_xy[jj], c = s_zq[jj], d = s_ok[jj];
+      const long long jg = jt * kVvTile + jj;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        if (jg >= i[k]) continue;
+        const VvPair v = vv_pair(p[k], a, c, d);
+        vv_add(p[k], v, c.y, recip(v.den));
+      }
+    }
   }
+  double *out = part + 3 * (long long)seg * npts;
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (i[k] < npts) {
+      out[i[k]] = live[k] ? p[k].f * -1.5 : 0.0;
+      out[npts + i[k]] = live[k] ? p[k].u : 0.0;
+      out[2 * npts + i[k]] = live[k] ? p[k].w : 0.0;
+    }
 }
 
 // input order -> leaf order: weighted exc, vrho, vsigma (nonlocal_correlation.
@@ -170,7 +276,8 @@ __global__ __launch_bounds__(256) void k_vv10_pairs(double *__restrict__ nlc, lo
 // 295-303).  A point with rho < 1e-8 keeps exc = vrho = beta w, vsigma = 0.
 __global__ __launch_bounds__(256) void k_vv10_coef(BuildArgs a, const double *__restrict__ rho4,
                                                    const int *__restrict__ porig, Vv10Consts k,
-                                                   const double *__restrict__ nlc, long long npts) {
+                                                   const double *__restrict__ part, long long npts,
+                                                   int seg_tiles) {
   __shared__ double s_red[4];
   const int leaf = blockIdx.x;
   const LeafDev L = a.leaves[leaf];
@@ -192,7 +299,15 @@ __global__ __launch_bounds__(256) void k_vv10_coef(BuildArgs a, const double *__
       const double dom_dr = (0.5 * pi4_3 * rho - 2.0 * tmp) / om;
       const double dom_dg = sigma > 0.0 ? tmp * rho / (sigma * om) : 0.0;
       const double dka_dr = (1.0 / 6.0) * ka;
-      const double F = nlc[kF * npts + o], U = nlc[kU * npts + o], W = nlc[kW * npts + o];
+      // the segments that the point's block has, in order
+      double F = 0.0, U = 0.0, W = 0.0;
+      const int nseg = (int)((2 * (o / kVvRows) + 1) / seg_tiles) + 1;
+      for (int g = 0; g < nseg; ++g) {
+        const double *f = part + 3 * (long long)g * npts + o;
+        F += f[0];
+        U += f[npts];
+        W += f[2 * npts];
+      }
       ex = (k.beta + 0.5 * F) * w;
       vr = (k.beta + F + 1.5 * (U * dka_dr + W * dom_dr)) * w;
       vs = (1.5 * W * dom_dg) * w;
@@ -215,19 +330,24 @@ __global__ __launch_bounds__(256) void k_vv10_coef(BuildArgs a, const double *__
 
 } // namespace
 
-size_t nlc_buffer_elems(long long npts) { return (size_t)kNlcPlanes * (size_t)npts; }
+size_t nlc_buffer_elems(long long npts) {
+  return (size_t)(kNlcPlanes + 3 * vv_segs(npts).n) * (size_t)npts;
+}
 
 void launch_vv10(const BuildArgs &a, const double *rho4, const int *porig, double b, double C,
                  double *nlc, long long npts, hipStream_t s) {
   if (a.nleaves == 0 || npts == 0) return;
   const Vv10Consts k = vv10_consts(b, C);
-  launch_zero(nlc, (long long)kNlcPlanes * npts, s);
+  const VvSegs g = vv_segs(npts);
+  double *part = nlc + (size_t)kNlcPlanes * npts;
+  // points outside every leaf keep rho = 0 and so stay out of the sums
+  launch_zero(nlc + kRHO * npts, npts, s);
   k_vv10_prep<<<a.nleaves, 256, 0, s>>>(a, rho4, porig, k, nlc, npts);
   check("k_vv10_prep");
-  const long long nblk = (npts + kVvTile - 1) / kVvTile;
-  k_vv10_pairs<<<(unsigned)nblk, kVvTile, 0, s>>>(nlc, npts);
+  const long long nblk = (npts + kVvRows - 1) / kVvRows;
+  k_vv10_pairs<<<dim3((unsigned)nblk, g.n), 256, 0, s>>>(nlc, npts, g.tiles, part);
   check("k_vv10_pairs");
-  k_vv10_coef<<<a.nleaves, 256, 0, s>>>(a, rho4, porig, k, nlc, npts);
+  k_vv10_coef<<<a.nleaves, 256, 0, s>>>(a, rho4, porig, k, part, npts, g.tiles);
   check("k_vv10_coef");
 }
 

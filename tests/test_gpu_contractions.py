@@ -98,3 +98,25 @@ def test_gradients_match_oracle(system, basis_name, method, precision):
     got = ctx.xc_gradient_unrestricted(Du, basis.shell_atom, n)
     assert np.abs(got - Gu).max() <= tol * max(1.0, np.abs(Gu).max())
     ctx.close()
+
+
+# VV10: one pass over several segments of j, points within and beyond the range
+# whose pairs share a reciprocal (atoms 1500 Bohr apart, a tiny b).  The sums run
+# in another order than the oracle's: 1e-12 of E; Vxc as a build's, plus the
+# rounding of 1e4 pair terms relative to its largest entry.
+@pytest.mark.parametrize("shift,b", [(0.0, 6.0), (1500.0, 6.0), (0.0, 1e-6), (3.0, 1e-9)])
+@pytest.mark.parametrize("nrad,nang", [(8, 26), (40, 50)])
+def test_vv10_matches_oracle(shift, b, nrad, nang):
+    atoms = molecules.water()
+    if shift:
+        atoms = atoms + [(z, x + shift, y, w) for z, x, y, w in molecules.water()]
+    basis = AOBasis.load(atoms, "6-31g")
+    pts, wts = MolecularGrid(atoms, GridSettings(radial_points=nrad, angular_points=nang)).build()
+    print(f"vv10 shift {shift} b {b} npts={len(wts)}", flush=True)
+    D = random_density(basis.nbf, 5, 41)
+    e, V = oracle.vv10(oracle.OracleBasis.from_flat(basis.flat()), pts, wts, D, b=b, C=0.01)
+    ctx = XCContext(basis, pts, wts, functional_ids("pbe"))
+    got, K = ctx.nlc_vv10(D, b=b, C=0.01)
+    ctx.close()
+    assert abs(got - e) <= 1e-12 * abs(e)
+    assert np.abs(K - V).max() <= 1e-11 + 1e-11 * np.abs(V).max()
