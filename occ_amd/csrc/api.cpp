@@ -662,7 +662,8 @@ void context_setup(occxc_context *c, int nmol, const occxc_basis *bases,
   const size_t nn = (size_t)c->mtot;
   c->d_D.alloc(nn);
   c->d_D2.alloc(nn);
-  c->d_K.alloc(nn);
+  c->k_rep = k_copies(c->mtot);
+  c->d_K.alloc(nn * c->k_rep);
   c->d_V.alloc(nn);
   c->d_coef.alloc((size_t)4 * std::max<long long>(c->ptot, 1));
   c->d_part.alloc((size_t)2 * std::max(c->nleaves, 1));
@@ -695,6 +696,7 @@ void context_setup(occxc_context *c, int nmol, const occxc_basis *bases,
   a.pw = c->d_pw.get();
   a.D2 = c->d_D2.get();
   a.K = c->d_K.get();
+  a.k_mask = c->k_rep - 1;
   a.coef = c->d_coef.get();
   a.coef_planes = 4;
   a.coef_tau_planes = 0;
@@ -768,7 +770,7 @@ void context_setup(occxc_context *c, int nmol, const occxc_basis *bases,
     a.ntchunks = (int)tchunks.size();
     a.tpartial = c->d_tpartial.get();
   }
-  c->device_bytes = ao_bytes + ds_bytes + c->d_D.bytes() * 4 + c->d_coef.bytes() + c->d_px.bytes() * 4 +
+  c->device_bytes = ao_bytes + ds_bytes + c->d_D.bytes() * 3 + c->d_K.bytes() + c->d_coef.bytes() + c->d_px.bytes() * 4 +
                     c->d_porig.bytes() +
                     c->d_ao_map.bytes() + c->d_leaves.bytes() + c->d_leaf_shells.bytes() +
                     c->plan.bytes + c->d_kloc.bytes() + c->d_tpairs.bytes() +
@@ -914,8 +916,8 @@ static void run_build_mgga(occxc_context *c, const double *d_D, double *d_V, dou
   const int prec = c->opt.precision;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf, s);
-    launch_zero(c->d_K.get(), c->mtot, s);
+    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf,
+                           c->d_K.get(), c->k_rep, c->mtot, s);
   });
   t.run(OCCXC_STAGE_DENSITY, [&] { mgga_density(c, s); });
   t.run(OCCXC_STAGE_VXC, [&] {
@@ -925,8 +927,8 @@ static void run_build_mgga(occxc_context *c, const double *d_D, double *d_V, dou
     run_vxc_mgga(c->plan, x, c->d_leaves_k.get(), c->d_ao.get(), prec, s);
   });
   t.run(OCCXC_STAGE_FINALIZE, [&] {
-    launch_finalize(c->d_K.get(), d_V, c->d_mols.get(), c->nmol, c->maxnbf, c->d_part.get(),
-                    d_result, s);
+    launch_finalize(c->d_K.get(), d_V, c->d_mols.get(), c->nmol, c->maxnbf, c->k_rep, c->mtot,
+                    c->d_part.get(), d_result, s);
     storage_correction(c, d_result, s);
   });
 }
@@ -940,8 +942,8 @@ void run_build(occxc_context *c, const double *d_D, double *d_V, double *d_resul
   const BuildArgs &a = c->args;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf, s);
-    if (!c->plan.two_pass) launch_zero(c->d_K.get(), c->mtot, s);
+    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf,
+                           c->plan.two_pass ? nullptr : c->d_K.get(), c->k_rep, c->mtot, s);
   });
   if (!c->plan.use_mfma) {
     const bool fp32 = c->opt.precision != OCCXC_PREC_FP64;
@@ -956,8 +958,8 @@ void run_build(occxc_context *c, const double *d_D, double *d_V, double *d_resul
       run_vxc_reduce(a, d_V, s);
       launch_finalize_scalars(c->d_mols.get(), c->nmol, c->d_part.get(), d_result, s);
     } else {
-      launch_finalize(c->d_K.get(), d_V, c->d_mols.get(), c->nmol, c->maxnbf, c->d_part.get(),
-                      d_result, s);
+      launch_finalize(c->d_K.get(), d_V, c->d_mols.get(), c->nmol, c->maxnbf, c->k_rep, c->mtot,
+                      c->d_part.get(), d_result, s);
     }
     storage_correction(c, d_result, s);
   });
@@ -973,8 +975,8 @@ static void run_nlc(occxc_context *c, const double *d_D, double b, double C, dou
   const int prec = c->opt.precision;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf, s);
-    if (!c->plan.two_pass) launch_zero(c->d_K.get(), c->mtot, s);
+    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf,
+                           c->plan.two_pass ? nullptr : c->d_K.get(), c->k_rep, c->mtot, s);
   });
   t.run(OCCXC_STAGE_DENSITY, [&] {
     BuildArgs x = a;
@@ -990,8 +992,8 @@ static void run_nlc(occxc_context *c, const double *d_D, double b, double C, dou
       run_vxc_reduce(a, d_V, s);
       launch_finalize_scalars(c->d_mols.get(), c->nmol, c->d_part.get(), d_result, s);
     } else {
-      launch_finalize(c->d_K.get(), d_V, c->d_mols.get(), c->nmol, c->maxnbf, c->d_part.get(),
-                      d_result, s);
+      launch_finalize(c->d_K.get(), d_V, c->d_mols.get(), c->nmol, c->maxnbf, c->k_rep, c->mtot,
+                      c->d_part.get(), d_result, s);
     }
   });
 }
@@ -1066,7 +1068,8 @@ void run_gradient(occxc_context *c, const double *d_D, double *d_grad, hipStream
   const BuildArgs &a = c->args;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf, s);
+    launch_prepare_density(d_D, c->d_D2.get(), c->d_mols.get(), c->nmol, c->maxnbf, nullptr, 0, 0,
+                           s);
   });
   t.run(OCCXC_STAGE_DENSITY, [&] {
     if (c->mgga)
@@ -1092,7 +1095,7 @@ void run_gradient(occxc_context *c, const double *d_D, double *d_grad, hipStream
   });
 }
 
-// Unrestricted build on stream s from the raw density in d_Du:
+// Unrestricted build on stream s from the raw density d_D:
 // compute_K_dft<d, Unrestricted> (dft.h:190-388).  Each spin density is
 // contracted by the density kernel in store mode, the polarised functional
 // stage forms both spins' coefficients, and the Vxc kernels run once per spin.
@@ -1119,18 +1122,16 @@ static void mgga_density_u(occxc_context *c, hipStream_t s) {
                                     c->d_part_u.get(), s);
 }
 
-void run_build_u(occxc_context *c, hipStream_t s) {
+void run_build_u(occxc_context *c, const double *d_D, double *d_V, double *d_result,
+                 hipStream_t s) {
   const BuildArgs &a = c->args;
   const int prec = c->opt.precision;
   const bool two_pass = c->plan.two_pass;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
-                             c->d_D2sb.get(), c->nbf, s);
-    if (!two_pass) {
-      launch_zero(c->d_K.get(), c->mtot, s);
-      launch_zero(c->d_K_b.get(), c->mtot, s);
-    }
+    launch_prepare_density_u(d_D, c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
+                             c->d_D2sb.get(), c->nbf, two_pass ? nullptr : c->d_K.get(),
+                             c->d_K_b.get(), c->k_rep, s);
   });
   if (c->mgga) {
     t.run(OCCXC_STAGE_DENSITY, [&] { mgga_density_u(c, s); });
@@ -1166,27 +1167,33 @@ void run_build_u(occxc_context *c, hipStream_t s) {
   });
   }
   t.run(OCCXC_STAGE_FINALIZE, [&] {
-    launch_finalize_u(two_pass ? nullptr : c->d_K.get(), c->d_K_b.get(), c->d_V.get(),
-                      c->d_V_b.get(), c->d_mols.get(), c->maxnbf, c->d_part_u.get(),
-                      c->nleaves, c->d_result_u.get(), s);
+    if (two_pass) {
+      const size_t row = (size_t)c->nbf * sizeof(double);
+      OCCXC_HIP(hipMemcpy2DAsync(d_V, 2 * row, c->d_V.get(), row, row, c->nbf,
+                                 hipMemcpyDeviceToDevice, s));
+      OCCXC_HIP(hipMemcpy2DAsync(d_V + c->nbf, 2 * row, c->d_V_b.get(), row, row, c->nbf,
+                                 hipMemcpyDeviceToDevice, s));
+    }
+    launch_finalize_u(two_pass ? nullptr : c->d_K.get(), c->d_K_b.get(), d_V, c->nbf, c->k_rep,
+                      c->d_part_u.get(), c->nleaves, d_result, s);
   });
 }
 
 void uks_setup(occxc_context *c);
 
-// Unrestricted XC gradient on stream s from the raw density in d_Du: both
+// Unrestricted XC gradient on stream s from the raw density d_D: both
 // spin densities and the polarised functional stage as in run_build_u, then
 // the gradient partials once per spin (P_s = 2 D_s, that spin's
 // coefficients) and one per-atom reduction of both
 // (process_grid_block_gradient<d, Unrestricted>, dft_gradient_kernels.cpp:
 // 473-583).
-void run_gradient_u(occxc_context *c, double *d_grad, hipStream_t s) {
+void run_gradient_u(occxc_context *c, const double *d_D, double *d_grad, hipStream_t s) {
   const BuildArgs &a = c->args;
   const int prec = c->opt.precision;
   StageTimer t{c, s, {}};
   t.run(OCCXC_STAGE_PREPARE, [&] {
-    launch_prepare_density_u(c->d_Du.get(), c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
-                             c->d_D2sb.get(), c->nbf, s);
+    launch_prepare_density_u(d_D, c->d_D2a.get(), c->d_D2b.get(), c->d_D2sa.get(),
+                             c->d_D2sb.get(), c->nbf, nullptr, nullptr, 0, s);
   });
   t.run(OCCXC_STAGE_DENSITY, [&] {
     if (c->mgga) {
@@ -1228,17 +1235,17 @@ void run_gradient_u(occxc_context *c, double *d_grad, hipStream_t s) {
 void uks_setup(occxc_context *c) {
   if (c->uks_ready) return;
   const size_t nn = (size_t)c->nbf * c->nbf;
-  c->d_Du.alloc(2 * nn);
   c->d_D2a.alloc(nn);
   c->d_D2b.alloc(nn);
   c->d_rho_a.alloc(4 * (size_t)c->ptot);
   c->d_rho_b.alloc(4 * (size_t)c->ptot);
   c->d_coef_b.alloc(4 * (size_t)c->ptot);
-  c->d_K_b.alloc(nn);
-  c->d_V_b.alloc(nn);
+  c->d_K_b.alloc(nn * c->k_rep);
+  if (c->plan.two_pass) c->d_V_b.alloc(nn);
   c->d_part_u.alloc(3 * (size_t)std::max(c->nleaves, 1));
   c->d_result_u.alloc(3);
-  c->device_bytes += 8.0 * (7 * nn + 12 * (size_t)c->ptot + 3 * (size_t)c->nleaves + 3);
+  c->device_bytes += 8.0 * (2 * nn + 12 * (size_t)c->ptot + 3 * (size_t)c->nleaves + 3) +
+                     c->d_K_b.bytes() + c->d_V_b.bytes();
   if (c->mgga) {
     c->d_mtau_b.alloc(3 * (size_t)c->ptot);
     c->d_coef_tau_b.alloc(c->ptot);
@@ -1247,6 +1254,15 @@ void uks_setup(occxc_context *c) {
     c->device_bytes += 8.0 * (4 * (size_t)c->ptot + 2 * nn);
   }
   c->uks_ready = true;
+}
+
+// Device copies of D and Vxc (2 nbf x nbf) for the host entry points.
+void uks_host_buffers(occxc_context *c) {
+  if (c->d_Du.size()) return;
+  const size_t nn = (size_t)c->nbf * c->nbf;
+  c->d_Du.alloc(2 * nn);
+  c->d_Vu.alloc(2 * nn);
+  c->device_bytes += c->d_Du.bytes() + c->d_Vu.bytes();
 }
 
 void drop_graph(occxc_context *c) {
@@ -1550,13 +1566,10 @@ occxc_status occxc_build_unrestricted(occxc_context *ctx, const double *D, doubl
       OCCXC_REQUIRE(std::isfinite(D[i]), OCCXC_ERR_INVALID_ARGUMENT, "D: non-finite entry");
     DeviceGuard g(ctx->device);
     uks_setup(ctx);
+    uks_host_buffers(ctx);
     ctx->d_Du.upload(D, 2 * nn, ctx->stream);
-    run_build_u(ctx, ctx->stream);
-    const size_t row = (size_t)ctx->nbf * sizeof(double);
-    OCCXC_HIP(hipMemcpy2DAsync(Vxc, 2 * row, ctx->d_V.get(), row, row, ctx->nbf,
-                               hipMemcpyDeviceToHost, ctx->stream));
-    OCCXC_HIP(hipMemcpy2DAsync(Vxc + ctx->nbf, 2 * row, ctx->d_V_b.get(), row, row, ctx->nbf,
-                               hipMemcpyDeviceToHost, ctx->stream));
+    run_build_u(ctx, ctx->d_Du.get(), ctx->d_Vu.get(), ctx->d_result_u.get(), ctx->stream);
+    ctx->d_Vu.download(Vxc, 2 * nn, ctx->stream);
     double r[3];
     ctx->d_result_u.download(r, 3, ctx->stream);
     OCCXC_HIP(hipStreamSynchronize(ctx->stream));
@@ -1582,17 +1595,7 @@ occxc_status occxc_build_unrestricted_device(occxc_context *ctx, const double *d
     DeviceGuard g(ctx->device);
     uks_setup(ctx);
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
-    const size_t nn = (size_t)ctx->nbf * ctx->nbf;
-    OCCXC_HIP(hipMemcpyAsync(ctx->d_Du.get(), d_D, 2 * nn * sizeof(double),
-                             hipMemcpyDeviceToDevice, s));
-    run_build_u(ctx, s);
-    const size_t row = (size_t)ctx->nbf * sizeof(double);
-    OCCXC_HIP(hipMemcpy2DAsync(d_Vxc, 2 * row, ctx->d_V.get(), row, row, ctx->nbf,
-                               hipMemcpyDeviceToDevice, s));
-    OCCXC_HIP(hipMemcpy2DAsync(d_Vxc + ctx->nbf, 2 * row, ctx->d_V_b.get(), row, row, ctx->nbf,
-                               hipMemcpyDeviceToDevice, s));
-    OCCXC_HIP(hipMemcpyAsync(d_result, ctx->d_result_u.get(), 3 * sizeof(double),
-                             hipMemcpyDeviceToDevice, s));
+    run_build_u(ctx, d_D, d_Vxc, d_result, s);
   });
 }
 
@@ -1630,8 +1633,9 @@ occxc_status occxc_xc_gradient_unrestricted(occxc_context *ctx, const double *D,
       OCCXC_REQUIRE(std::isfinite(D[i]), OCCXC_ERR_INVALID_ARGUMENT, "D: non-finite entry");
     DeviceGuard g(ctx->device);
     gradient_u_prepare(ctx, natoms, shell_atom);
+    uks_host_buffers(ctx);
     ctx->d_Du.upload(D, 2 * nn, ctx->stream);
-    run_gradient_u(ctx, ctx->d_grad.get(), ctx->stream);
+    run_gradient_u(ctx, ctx->d_Du.get(), ctx->d_grad.get(), ctx->stream);
     ctx->d_grad.download(grad, 3 * (size_t)natoms, ctx->stream);
     OCCXC_HIP(hipStreamSynchronize(ctx->stream));
   });
@@ -1646,10 +1650,7 @@ occxc_status occxc_xc_gradient_unrestricted_device(occxc_context *ctx, const dou
     DeviceGuard g(ctx->device);
     gradient_u_prepare(ctx, natoms, shell_atom);
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
-    const size_t nn = (size_t)ctx->nbf * ctx->nbf;
-    OCCXC_HIP(hipMemcpyAsync(ctx->d_Du.get(), d_D, 2 * nn * sizeof(double),
-                             hipMemcpyDeviceToDevice, s));
-    run_gradient_u(ctx, d_grad, s);
+    run_gradient_u(ctx, d_D, d_grad, s);
   });
 }
 

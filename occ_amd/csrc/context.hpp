@@ -43,6 +43,7 @@ struct occxc_context {
   occxc::DevBuf<float> d_ao_res;
   occxc::DevBuf<float> d_ao_a;  // FP32 mode: the Vxc stage's A plane (A pass)
   occxc::DevBuf<double> d_dS, d_ncorr;
+  int k_rep = 1;  // copies of K (k_copies)
   occxc::DevBuf<double> d_D, d_D2, d_K, d_V, d_coef, d_part, d_result;
   occxc::ContractPlan plan;
   // two-pass Vxc: per-leaf K_loc blocks and the tile-pair leaf lists
@@ -77,11 +78,12 @@ struct occxc_context {
   bool ao2_ready = false;
   std::vector<int> grad_shell_atom;
   int grad_natoms = 0;
-  // unrestricted builds (allocated on the first one): the raw 2 nbf x nbf
-  // density, 2 D_s^T per spin, rho and grad rho per spin, the beta-spin
-  // coefficients and K / Vxc (alpha uses the restricted buffers), per-leaf
-  // {Exc, N_alpha, N_beta} and the result {Exc, N_alpha, N_beta}
-  occxc::DevBuf<double> d_Du, d_D2a, d_D2b, d_rho_a, d_rho_b, d_coef_b, d_K_b, d_V_b, d_part_u,
+  // unrestricted builds (allocated on the first one): 2 D_s^T per spin, rho and
+  // grad rho per spin, the beta-spin coefficients and K (alpha uses the
+  // restricted buffers; d_V_b in the two-pass form only), per-leaf {Exc,
+  // N_alpha, N_beta} and the result; for the host entry points D and Vxc
+  // (2 nbf x nbf)
+  occxc::DevBuf<double> d_Du, d_Vu, d_D2a, d_D2b, d_rho_a, d_rho_b, d_coef_b, d_K_b, d_V_b, d_part_u,
       d_result_u;
   bool uks_ready = false;
   // restricted meta-GGA (allocated at context creation): rho and grad rho

@@ -2422,7 +2422,7 @@ __global__ __launch_bounds__(256, 2) void k_vxc_gemm_f32(BuildArgs a, const floa
   if (it.leaf < 0 || !a.leaf_active[it.leaf]) return;
   const LeafDev L = a.leaves[it.leaf];
   const MolDev MD = a.mols[L.mol];
-  double *Km = a.K + MD.moff;
+  double *Km = a.K + MD.moff + (it.leaf & a.k_mask) * a.mtot;
   const int *map = ao_map + L.map_off;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -2546,7 +2546,7 @@ __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__rest
   constexpr int NH = PT / 8;  // operand rounds of 8 points per chunk
   const LeafDev L = a.leaves[it.leaf];
   const MolDev MD = a.mols[L.mol];
-  double *Km = a.K + MD.moff;
+  double *Km = a.K + MD.moff + (it.leaf & a.k_mask) * a.mtot;
   const int *map = ao_map + L.map_off;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);

@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void k_density_functional(BuildArgs a,
 
 // ---------------------------------------------------------------- Vxc --
 // K_loc(mu, nu) = sum_p phi(p,mu) A(p,nu),  A = c0 phi + c . grad phi,
-// scattered into K with FP64 atomics; Vxc = K + K^T in k_finalize_matrix.
+// scattered into K with FP64 atomics; Vxc = K + K^T in k_finalize.
 template <typename T>
 __global__ __launch_bounds__(256) void k_vxc(BuildArgs a, const T *__restrict__ ao) {
   __shared__ int s_map[kMaxLocalAo];
@@ -532,9 +532,11 @@ __global__ void k_zero(double *__restrict__ p, long long n) {
     p[k] = 0.0;
 }
 
-// blockIdx.y = molecule; D2 = 2 D with the upper triangle mirrored
+// blockIdx.y = molecule; D2 = 2 D with the upper triangle mirrored, and the
+// nrep copies of K (mtot apart; none when K is null) cleared
 __global__ void k_prepare_density(const double *__restrict__ D, double *__restrict__ D2,
-                                  const MolDev *__restrict__ mols) {
+                                  const MolDev *__restrict__ mols, double *__restrict__ K,
+                                  int nrep, long long mtot) {
   const MolDev M = mols[blockIdx.y];
   const int nbf = M.nbf;
   const long long n = (long long)nbf * nbf;
@@ -544,19 +546,21 @@ __global__ void k_prepare_density(const double *__restrict__ D, double *__restri
     const int i = (int)(k % nbf), j = (int)(k / nbf);
     const int r = i < j ? i : j, c = i < j ? j : i;
     D2[M.moff + k] = 2.0 * Dm[r + (long long)c * nbf];
+    if (K)
+      for (int y = 0; y < nrep; ++y) K[M.moff + k + y * mtot] = 0.0;
   }
 }
 
-// blockIdx.y = molecule; Vxc = K + K^T
-// V = K + K^T
 // Unrestricted D (2 nbf x nbf, alpha rows over beta rows, one molecule):
 // D2t_s = 2 D_s^T for each spin, the full block (evaluate_density<d, U> uses
 // no selfadjointView, density.cpp:18-30,45-70); the contraction kernels read
 // D2t(nu, mu) as D2(mu, nu).  D2sa / D2sb (null unless a meta-GGA): D_s + D_s^T,
-// exactly symmetric, which gives the tau row sums of 2 D_s.
+// exactly symmetric, which gives the tau row sums of 2 D_s.  The nrep copies
+// of both spins' K are cleared (none when Ka is null).
 __global__ void k_prepare_density_u(const double *__restrict__ D, double *__restrict__ D2a,
                                     double *__restrict__ D2b, double *__restrict__ D2sa,
-                                    double *__restrict__ D2sb, int nbf) {
+                                    double *__restrict__ D2sb, int nbf,
+                                    double *__restrict__ Ka, double *__restrict__ Kb, int nrep) {
   const long long n = (long long)nbf * nbf;
   for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n;
        k += (long long)gridDim.x * blockDim.x) {
@@ -568,6 +572,8 @@ __global__ void k_prepare_density_u(const double *__restrict__ D, double *__rest
       D2sa[k] = da + D[nu + (long long)mu * 2 * nbf];
       D2sb[k] = db + D[nbf + nu + (long long)mu * 2 * nbf];
     }
+    if (Ka)
+      for (int y = 0; y < nrep; ++y) Ka[k + y * n] = Kb[k + y * n] = 0.0;
   }
 }
 
@@ -773,19 +779,6 @@ __global__ void k_functional_mgga_points(int id, long long n, const double *__re
 }
 
 // {Exc, N_alpha, N_beta}: fixed-order sums of the per-leaf partials
-__global__ __launch_bounds__(256) void k_finalize_scalars_u(const double *__restrict__ part,
-                                                            int nleaves,
-                                                            double *__restrict__ result) {
-  __shared__ double s_red[4];
-  double v[3] = {0, 0, 0};
-  for (int i = threadIdx.x; i < nleaves; i += 256)
-    for (int k = 0; k < 3; ++k) v[k] += part[3 * i + k];
-  for (int k = 0; k < 3; ++k) {
-    const double t = block_sum_256(v[k], s_red);
-    if (threadIdx.x == 0) result[k] = t;
-  }
-}
-
 // Polarised functionals over points (libxc layout), ADDING to the outputs.
 __global__ void k_functional_pol_points(int id, long long n, const double *__restrict__ rho,
                                         const double *__restrict__ sigma,
@@ -881,8 +874,8 @@ __global__ __launch_bounds__(256) void k_ncorr_final(const double *__restrict__ 
   if (threadIdx.x == 0) result[2 * blockIdx.x + 1] += t;
 }
 
-__global__ void k_finalize_matrix(const double *__restrict__ K, double *__restrict__ V,
-                                  const MolDev *__restrict__ mols) {
+__global__ void k_symmetrize(const double *__restrict__ K, double *__restrict__ V,
+                             const MolDev *__restrict__ mols) {
   const MolDev M = mols[blockIdx.y];
   const int nbf = M.nbf;
   const long long n = (long long)nbf * nbf;
@@ -894,22 +887,91 @@ __global__ void k_finalize_matrix(const double *__restrict__ K, double *__restri
   }
 }
 
+// result[q] = sum over the leaves [lo, hi) of part[NQ leaf + q], in a fixed
+// order: per-thread strided sums (eight leaves' loads in flight), then a fixed
+// tree.  One workgroup of 256.
+template <int NQ>
+__device__ void leaf_sums(const double *__restrict__ part, int lo, int hi, double *s_red,
+                          double *__restrict__ result) {
+  double v[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) v[q] = 0.0;
+  for (int i = lo + threadIdx.x; i < hi; i += 8 * 256) {
+    double x[8][NQ];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        x[u][q] = i + 256 * u < hi ? part[(long long)NQ * (i + 256 * u) + q] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) v[q] += x[u][q];
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const double t = block_sum_256(v[q], s_red);
+    if (threadIdx.x == 0) result[q] = t;
+  }
+}
+
 // one workgroup per molecule: {Exc, N_elec} over its leaves in a fixed order
 __global__ __launch_bounds__(256) void k_finalize_scalars(const double *__restrict__ part,
                                                           const MolDev *__restrict__ mols,
                                                           double *__restrict__ result) {
   __shared__ double s_red[4];
   const MolDev M = mols[blockIdx.x];
-  double e = 0.0, n = 0.0;
-  for (int i = M.leaf_begin + threadIdx.x; i < M.leaf_end; i += 256) {
-    e += part[2 * i];
-    n += part[2 * i + 1];
+  leaf_sums<2>(part, M.leaf_begin, M.leaf_end, s_red, result + 2 * blockIdx.x);
+}
+
+// Vxc = K + K^T, K the sum of its nrep copies (mtot apart), and the scalars,
+// in one launch: block (0, molecule) the scalars, the others the matrix.
+__global__ __launch_bounds__(256) void k_finalize(const double *__restrict__ K,
+                                                  double *__restrict__ V,
+                                                  const MolDev *__restrict__ mols, int nrep,
+                                                  long long mtot, const double *__restrict__ part,
+                                                  double *__restrict__ result) {
+  __shared__ double s_red[4];
+  const MolDev M = mols[blockIdx.y];
+  if (blockIdx.x == 0) {
+    leaf_sums<2>(part, M.leaf_begin, M.leaf_end, s_red, result + 2 * blockIdx.y);
+    return;
   }
-  e = block_sum_256(e, s_red);
-  n = block_sum_256(n, s_red);
-  if (threadIdx.x == 0) {
-    result[2 * blockIdx.x] = e;
-    result[2 * blockIdx.x + 1] = n;
+  const int nbf = M.nbf;
+  const long long n = (long long)nbf * nbf;
+  const double *Km = K + M.moff;
+  for (long long k = (blockIdx.x - 1) * (long long)blockDim.x + threadIdx.x; k < n;
+       k += (long long)(gridDim.x - 1) * blockDim.x) {
+    const int i = (int)(k % nbf), j = (int)(k / nbf);
+    const long long kt = j + (long long)i * nbf;
+    double v = Km[k] + Km[kt];
+    for (int y = 1; y < nrep; ++y) v += Km[k + y * mtot] + Km[kt + y * mtot];
+    V[M.moff + k] = v;
+  }
+}
+
+// The same for an unrestricted build of one molecule: blockIdx.y = spin, V 2nbf
+// x nbf (alpha rows over beta rows), {Exc, N_alpha, N_beta}.  Without Ka only
+// the scalars (block (0, 0)).
+__global__ __launch_bounds__(256) void k_finalize_u(const double *__restrict__ Ka,
+                                                    const double *__restrict__ Kb,
+                                                    double *__restrict__ V, int nbf, int nrep,
+                                                    const double *__restrict__ part, int nleaves,
+                                                    double *__restrict__ result) {
+  __shared__ double s_red[4];
+  if (blockIdx.x == 0) {
+    if (blockIdx.y == 0) leaf_sums<3>(part, 0, nleaves, s_red, result);
+    return;
+  }
+  const double *K = blockIdx.y ? Kb : Ka;
+  const long long n = (long long)nbf * nbf;
+  for (long long k = (blockIdx.x - 1) * (long long)blockDim.x + threadIdx.x; k < n;
+       k += (long long)(gridDim.x - 1) * blockDim.x) {
+    const int i = (int)(k % nbf), j = (int)(k / nbf);
+    const long long kt = j + (long long)i * nbf;
+    double v = K[k] + K[kt];
+    for (int y = 1; y < nrep; ++y) v += K[k + y * n] + K[kt + y * n];
+    V[(long long)j * 2 * nbf + blockIdx.y * nbf + i] = v;
   }
 }
 
@@ -1106,9 +1168,9 @@ static dim3 mol_grid(int maxnbf, int nmol) {
 }
 
 void launch_prepare_density(const double *D, double *D2, const MolDev *mols, int nmol,
-                            int maxnbf, hipStream_t s) {
+                            int maxnbf, double *K, int nrep, long long mtot, hipStream_t s) {
   if (nmol == 0) return;
-  k_prepare_density<<<mol_grid(maxnbf, nmol), 256, 0, s>>>(D, D2, mols);
+  k_prepare_density<<<mol_grid(maxnbf, nmol), 256, 0, s>>>(D, D2, mols, K, nrep, mtot);
   check_launch();
 }
 
@@ -1174,10 +1236,11 @@ void launch_finalize_scalars(const MolDev *mols, int nmol, const double *leaf_pa
 }
 
 void launch_prepare_density_u(const double *D, double *D2a, double *D2b, double *D2sa,
-                              double *D2sb, int nbf, hipStream_t s) {
+                              double *D2sb, int nbf, double *Ka, double *Kb, int nrep,
+                              hipStream_t s) {
   const long long n = (long long)nbf * nbf;
   if (n == 0) return;
-  k_prepare_density_u<<<grid_for(n, 256), 256, 0, s>>>(D, D2a, D2b, D2sa, D2sb, nbf);
+  k_prepare_density_u<<<grid_for(n, 256), 256, 0, s>>>(D, D2a, D2b, D2sa, D2sb, nbf, Ka, Kb, nrep);
   check_launch();
 }
 
@@ -1214,16 +1277,10 @@ void launch_functional_mgga(int id, long long n, const double *rho, const double
   check_launch();
 }
 
-void launch_finalize_u(const double *Ka, const double *Kb, double *Va, double *Vb,
-                       const MolDev *mols, int maxnbf, const double *part, int nleaves,
-                       double *result, hipStream_t s) {
-  if (Ka) {
-    k_finalize_matrix<<<mol_grid(maxnbf, 1), 256, 0, s>>>(Ka, Va, mols);
-    check_launch();
-    k_finalize_matrix<<<mol_grid(maxnbf, 1), 256, 0, s>>>(Kb, Vb, mols);
-    check_launch();
-  }
-  k_finalize_scalars_u<<<1, 256, 0, s>>>(part, nleaves, result);
+void launch_finalize_u(const double *Ka, const double *Kb, double *V, int nbf, int nrep,
+                       const double *part, int nleaves, double *result, hipStream_t s) {
+  const dim3 g = Ka ? dim3(mol_grid(nbf, 1).x + 1, 2) : dim3(1, 1);
+  k_finalize_u<<<g, 256, 0, s>>>(Ka, Kb, V, nbf, nrep, part, nleaves, result);
   check_launch();
 }
 
@@ -1246,7 +1303,7 @@ void launch_functional_mgga_pol(int id, long long n, const double *rho, const do
 void launch_symmetrize(const double *K, double *out, const MolDev *mols, int nmol, int maxnbf,
                        hipStream_t s) {
   if (nmol == 0) return;
-  k_finalize_matrix<<<mol_grid(maxnbf, nmol), 256, 0, s>>>(K, out, mols);
+  k_symmetrize<<<mol_grid(maxnbf, nmol), 256, 0, s>>>(K, out, mols);
   check_launch();
 }
 
@@ -1263,11 +1320,11 @@ void launch_storage_correction(const double *D2, const double *dS, const MolDev 
 }
 
 void launch_finalize(const double *K, double *Vxc, const MolDev *mols, int nmol, int maxnbf,
-                     const double *leaf_part, double *result, hipStream_t s) {
+                     int nrep, long long mtot, const double *leaf_part, double *result,
+                     hipStream_t s) {
   if (nmol == 0) return;
-  k_finalize_matrix<<<mol_grid(maxnbf, nmol), 256, 0, s>>>(K, Vxc, mols);
-  check_launch();
-  k_finalize_scalars<<<nmol, 256, 0, s>>>(leaf_part, mols, result);
+  const dim3 g = mol_grid(maxnbf, nmol);
+  k_finalize<<<dim3(g.x + 1, g.y), 256, 0, s>>>(K, Vxc, mols, nrep, mtot, leaf_part, result);
   check_launch();
 }
 

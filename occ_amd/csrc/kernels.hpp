@@ -148,6 +148,7 @@ struct BuildArgs {
   const double *px, *py, *pz, *pw;
   const double *D2;     // doubled, symmetrised densities (concatenated nbf x nbf)
   double *K;            // accumulated phi^T A (concatenated nbf x nbf)
+  int k_mask;           // copies of K - 1: leaf l's items add into copy l & k_mask, mtot apart
   double *coef;         // per-point Vxc coefficients [4][ptot] (the density stage writes 4
                         // planes; the Vxc stage reads 4 for a GGA, 1 for an LDA)
   double *leaf_part;    // [2*nleaves] {Exc, N_elec} per leaf
@@ -211,8 +212,20 @@ constexpr int kNcorrBlocks = 1024;
 constexpr size_t kResidualChunkElems = (size_t)1 << 28;
 void launch_storage_correction(const double *D2, const double *dS, const MolDev *mols, int nmol,
                                int maxnbf, double *partial, double *result, hipStream_t s);
+// Copies of K that the Vxc items of a context with mtot matrix elements add
+// into, leaf l into copy l % k_copies: the atomics of many leaves on few
+// elements queue up per address (water / 6-31G: 531 leaves on 91 elements, 12 of
+// the Vxc kernel's 27 us).  The smallest matrices take 16 copies, those of
+// more than 16,384 elements (128 basis functions) one.
+inline int k_copies(long long mtot) {
+  int n = 1;
+  while (n < 16 && 2 * n * mtot <= 32768) n *= 2;
+  return n;
+}
+// D2 = 2 sym(D) per molecule; clears the nrep copies of K (mtot apart) unless K
+// is null
 void launch_prepare_density(const double *D, double *D2, const MolDev *mols, int nmol,
-                            int maxnbf, hipStream_t s);
+                            int maxnbf, double *K, int nrep, long long mtot, hipStream_t s);
 void launch_ao_eval(const BuildArgs &a, void *ao, bool fp32, hipStream_t s);
 // FP32 storage, context set-up: the value plane's rounding residuals of the
 // leaves [a.res_leaf0, a.res_leaf1) into a.ao_res (the stored values are not
@@ -241,18 +254,18 @@ void launch_grad_reduce(const double *gpart, const double *gpart2, int natoms,
 void launch_density_functional(const BuildArgs &a, const void *ao, bool fp32,
                                hipStream_t s);
 void launch_vxc(const BuildArgs &a, const void *ao, bool fp32, hipStream_t s);
-// unrestricted build (one molecule): D2t_s = 2 D_s^T and, when D2sa is given
-// (meta-GGA), D_s + D_s^T per spin; the polarised
-// functional stage per leaf (coef_a in a.coef, {Exc, N_a, N_b} per leaf in
-// part); V_s = K_s + K_s^T (skipped when Ka is null) and the fixed-order
-// scalar sums into result[3]
+// unrestricted build (one molecule): D2t_s = 2 D_s^T, D_s + D_s^T per spin when
+// D2sa is given (meta-GGA), and both spins' copies of K cleared (when Ka is
+// given); the polarised functional stage per leaf (coef_a in a.coef, {Exc, N_a,
+// N_b} per leaf in part); V_s = K_s + K_s^T into V (2 nbf x nbf; skipped when
+// Ka is null) and the fixed-order scalar sums into result[3]
 void launch_prepare_density_u(const double *D, double *D2a, double *D2b, double *D2sa,
-                              double *D2sb, int nbf, hipStream_t s);
+                              double *D2sb, int nbf, double *Ka, double *Kb, int nrep,
+                              hipStream_t s);
 void launch_functional_pol_leaves(const BuildArgs &a, const double *rho_a, const double *rho_b,
                                   double *coef_b, double *part, hipStream_t s);
-void launch_finalize_u(const double *Ka, const double *Kb, double *Va, double *Vb,
-                       const MolDev *mols, int maxnbf, const double *part, int nleaves,
-                       double *result, hipStream_t s);
+void launch_finalize_u(const double *Ka, const double *Kb, double *V, int nbf, int nrep,
+                       const double *part, int nleaves, double *result, hipStream_t s);
 void launch_functional_pol(int id, long long n, const double *rho, const double *sigma,
                            double *exc, double *vrho, double *vsigma, hipStream_t s);
 // polarised meta-GGA over points (ADDING; rho[2n], sigma[3n], tau[2n])
@@ -281,7 +294,8 @@ size_t nlc_buffer_elems(long long npts);
 void launch_vv10(const BuildArgs &a, const double *rho4, const int *porig, double b, double C,
                  double *nlc, long long npts, hipStream_t s);
 void launch_finalize(const double *K, double *Vxc, const MolDev *mols, int nmol,
-                     int maxnbf, const double *leaf_part, double *result, hipStream_t s);
+                     int maxnbf, int nrep, long long mtot, const double *leaf_part,
+                     double *result, hipStream_t s);
 // {Exc, N_elec} per molecule only (the two-pass Vxc writes Vxc itself)
 void launch_finalize_scalars(const MolDev *mols, int nmol, const double *leaf_part,
                              double *result, hipStream_t s);
