@@ -1496,6 +1496,21 @@ __device__ __forceinline__ void tile_shape_ext(int rt, int ct, F &&f) {
   else f(IntC<4>{}, IntC<4>{});
 }
 
+// The shapes of a wavefront with at most RM x CM tiles (blocks of at most 64
+// AOs have two column tiles, and two row tiles where rows are AOs).
+template <int RM, int CM, typename F>
+__device__ __forceinline__ void tile_shape_max(int rt, int ct, F &&f) {
+  if constexpr (CM == 4) {
+    tile_shape_ext(rt, ct, f);
+  } else {
+    static_assert(CM == 2, "two or four column tiles");
+    if (rt == 0 || ct == 0) f(IntC<0>{}, IntC<0>{});
+    else if (RM > 3 && rt == 4) f(IntC<RM>{}, IntC<2>{});
+    else if (RM > 2 && rt == 3) f(IntC<RM < 3 ? RM : 3>{}, IntC<2>{});
+    else f(IntC<2>{}, IntC<2>{});
+  }
+}
+
 // Two FP64 k-steps of acc[i][j] += X_i^T Y_j.  x and y point at this lane's
 // pair of operands in row tile 0 and column tile 0 ([row][k] layout, LD
 // doubles per row: tile i starts 16 i rows further).
@@ -1540,19 +1555,19 @@ __device__ __forceinline__ void mfma_f32_k4(f4 (&acc)[4][4], const float *x, con
 // The epilogue's first loads (row tile 0's first NJ column tiles: all four
 // with FP32 storage, two with FP64) can be issued before it
 // (den_epi_first_loads, during the last k-chunk's MFMAs) and passed in; PRE
-// says they were.
-template <typename S> struct DenEpiFirst {
+// says they were.  CM: column tiles of a wavefront (half the loads with two).
+template <typename S, int CM = 4> struct DenEpiFirst {
   using V = typename Vec4Of<S>::type;
-  static constexpr int NJ = sizeof(S) == 4 ? 4 : 2;  // column tiles per load round
+  static constexpr int NJ = (sizeof(S) == 4 ? 4 : 2) * CM / 4;  // column tiles per load round
   V f[NJ], fx[NJ], fy[NJ], fz[NJ];
 };
 
 // zero is 0, made opaque by the caller inside its last-chunk branch, so the
 // loads' addresses are formed there rather than hoisted out of the k-loop
 // (held across the loop, they spilled)
-template <typename S, bool GGA>
+template <typename S, bool GGA, int CM>
 __device__ __forceinline__ void den_epi_first_loads(const S *__restrict__ ao, const DenItem &it,
-                                                    const LeafDev &L, DenEpiFirst<S> &pre,
+                                                    const LeafDev &L, DenEpiFirst<S, CM> &pre,
                                                     int zero) {
   using V = typename Vec4Of<S>::type;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1564,7 +1579,7 @@ __device__ __forceinline__ void den_epi_first_loads(const S *__restrict__ ao, co
   const long long cs = (long long)L.mp * L.np;
   const int pl = wp * hp + 4 * g + zero;
 #pragma unroll
-  for (int j = 0; j < DenEpiFirst<S>::NJ; ++j) {
+  for (int j = 0; j < DenEpiFirst<S, CM>::NJ; ++j) {
     if (j >= CT) break;
     const long long off = (long long)(it.c0 + wc * hc + 16 * j + l16) * L.np + it.p0 + pl;
     pre.f[j] = *reinterpret_cast<const V *>(phi + off);
@@ -1579,12 +1594,13 @@ __device__ __forceinline__ void den_epi_first_loads(const S *__restrict__ ao, co
 // STORE: the sums of a leaf's only item go to a.rho_out (planes of ptot
 // doubles) instead of the functional; kq is the first quantity's plane there
 // and in the partial slots.
-template <typename S, bool GGA, bool PRE = false, bool STORE = false>
+template <typename S, bool GGA, bool PRE = false, bool STORE = false, int CM = 4>
 __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *__restrict__ ao,
                                                   const DenItem &it, const LeafDev &L,
-                                                  d4 (&acc)[4][4], double *__restrict__ part,
+                                                  d4 (&acc)[4][CM], double *__restrict__ part,
                                                   double *s_phi, double *s_red,
-                                                  const DenEpiFirst<S> *pre = nullptr, int kq = 0) {
+                                                  const DenEpiFirst<S, CM> *pre = nullptr,
+                                                  int kq = 0) {
   double(*s_q)[kMaxLeafPts] = reinterpret_cast<double(*)[kMaxLeafPts]>(s_phi);
   double(*s_h)[kTileAo] = reinterpret_cast<double(*)[kTileAo]>(s_phi + 4 * kMaxLeafPts);
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1608,9 +1624,9 @@ __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *_
     // NJ column tiles' loads in flight before any is used, kept as stored
     // (64 registers of loads: all four tiles with FP32 storage, two with FP64)
     using V = typename Vec4Of<S>::type;
-    constexpr int NJ = sizeof(S) == 4 ? 4 : 2;
+    constexpr int NJ = DenEpiFirst<S, CM>::NJ;
 #pragma unroll
-    for (int jj = 0; jj < 4; jj += NJ) {
+    for (int jj = 0; jj < CM; jj += NJ) {
       V f[NJ], fx[NJ], fy[NJ], fz[NJ];
 #pragma unroll
       for (int jq = 0; jq < NJ; ++jq) {
@@ -1801,13 +1817,18 @@ __device__ __forceinline__ void den_tile_item(const BuildArgs &a, const S *__res
 // the unused tiles read), so a chunk's loads are waited for by count.  The
 // MFMA k-step t reads AO 4 g + t of both, so the accumulators are those of
 // den_tile_item and the epilogue is shared.
-template <typename S> struct DenDma {
+// CW: the widest column block, 128 or, where a context's blocks are all at most
+// 64 AOs wide (small molecules), 64: half the accumulators and 24 KB (FP64)
+// buffers, so that three workgroups share a CU instead of two and the few
+// hundred items of a small molecule run in one round (water / 6-31G: 23.9 ->
+// 17.4 us; the Vxc items, four to a CU, 16.4 -> 12.8 us).
+template <typename S, int CW = kTileAo> struct DenDma {
   static constexpr int NS = sizeof(S) == 8 ? 2 : 3;               // LDS chunk buffers
   static constexpr int PHI = kTKc * kTileAo * (int)sizeof(S);     // bytes of Phi per buffer
-  static constexpr int STAGE = PHI + kTKc * kTileAo * 8;          // bytes per buffer
-  static constexpr int LOADS = (sizeof(S) == 8 ? 4 : 2) + 16;     // loads per chunk per wavefront
+  static constexpr int STAGE = PHI + kTKc * CW * 8;               // bytes per buffer
+  static constexpr int LOADS = (sizeof(S) == 8 ? 4 : 2) + CW / 8; // loads per chunk per wavefront
 };
-static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float>::STAGE / 8, "epilogue sums fit a stage");
+static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float, 64>::STAGE / 8, "epilogue sums fit a stage");
 
 // SYM (LDA form, symmetric D2): only the row sums of (Phi D2) o Phi are
 // wanted, so the k-loop of column block [c0, c0 + wc) stops at the block's end
@@ -1815,14 +1836,15 @@ static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float>::STAGE / 8, "epilog
 // the loads of a leaf of nb blocks go.
 // plane: the AO plane in Phi's place (1..3: the meta-GGA's tau passes, LDA
 // form), its sums going to quantity kq of the stored planes.
-template <typename S, bool GGA, bool SYM, bool STORE>
+template <typename S, bool GGA, bool SYM, bool STORE, int CW>
 __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *__restrict__ ao,
                                                   const int *__restrict__ ao_map,
                                                   const DenItem &it, double *__restrict__ part,
                                                   char *s_stage, double *s_red, int plane = 0,
                                                   int kq = 0) {
   static_assert(!(GGA && SYM), "grad rho needs all of Phi D2");
-  using P = DenDma<S>;
+  using P = DenDma<S, CW>;
+  constexpr int CM = CW / 32;  // column tiles of a wavefront
   LeafDev L = a.leaves[it.leaf];
   if constexpr (STORE && !GGA) L.ao_off += (long long)plane * L.mp * L.np;
   const MolDev MD = a.mols[L.mol];
@@ -1847,9 +1869,9 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
   // mirrors one triangle), so the row's entries are read along D2's
   // contiguous index: consecutive lanes, consecutive addresses wherever the
   // map is contiguous
-  long long colbase[4];
+  long long colbase[CM];
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb) colbase[cb] = map[it.c0 + min(32 * cb + (lane >> 1), it.wc - 1)];
+  for (int cb = 0; cb < CM; ++cb) colbase[cb] = map[it.c0 + min(32 * cb + (lane >> 1), it.wc - 1)];
   // Phi rows: 2 (FP64) or 4 (FP32) points per lane, clamped to the item's last ones
   constexpr int PPL = 16 / (int)sizeof(S);
   const int prow = sizeof(S) == 8 ? PPL * lane : PPL * (lane & 31);
@@ -1877,26 +1899,26 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
     }
     char *sd = st + P::PHI;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int kk = 4 * wave + (q >> 2), cb = q & 3;
+    for (int q = 0; q < 4 * CM; ++q) {
+      const int kk = 4 * wave + q / CM, cb = q % CM;
       __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const char *>(Dm + colbase[cb] + kmap[q >> 2]) + 4 * (lane & 1),
-          sd + (kk * kTileAo + 32 * cb) * 8, 4, 0, 0);
+          reinterpret_cast<const char *>(Dm + colbase[cb] + kmap[q / CM]) + 4 * (lane & 1),
+          sd + (kk * CW + 32 * cb) * 8, 4, 0, 0);
     }
   };
-  d4 acc[4][4];
+  d4 acc[4][CM];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int j = 0; j < CM; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   // AO chunks up to the leaf's real AOs (the padding rows of Phi are zero);
   // the wavefront's tiles that hold real points and real AO columns
   const int nch = ((SYM ? min(L.m, it.c0 + it.wc) : L.m) + kTKc - 1) / kTKc;
   const int cdbl = SYM && it.c0 > 0 ? it.c0 / kTKc : -1;  // first chunk of the block itself
   const int RTl = live_tiles(L.n - (it.p0 + wp * hp), hp), CTl = live_tiles(L.m - (it.c0 + wc * hc), hc);
-  DenEpiFirst<S> pre;
+  DenEpiFirst<S, CM> pre;
   for (int c = 0; c < P::NS - 1 && c < nch; ++c) dma(c * kTKc, s_stage + c * P::STAGE);
-  tile_shape_ext(RTl, CTl, [&](auto R, auto C) __attribute__((always_inline)) {
+  tile_shape_max<4, CM>(RTl, CTl, [&](auto R, auto C) __attribute__((always_inline)) {
     constexpr int NR = decltype(R)::value, NC = decltype(C)::value;
     int cur = 0;  // buffer of chunk c
     for (int c = 0; c < nch; ++c) {
@@ -1911,7 +1933,7 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
       if (c == nch - 1) {
         int zero = 0;
         asm volatile("" : "+s"(zero));  // an opaque 0: no instruction, no memory access
-        den_epi_first_loads<S, GGA>(ao, it, L, pre, zero);
+        den_epi_first_loads<S, GGA, CM>(ao, it, L, pre, zero);
       }
       const char *buf = s_stage + cur * P::STAGE;
       const S *sp = reinterpret_cast<const S *>(buf);
@@ -1930,7 +1952,7 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
 #pragma unroll
         for (int i = 0; i < NR; ++i) xv[i] = (double)sp[kk * kTileAo + wp * hp + 16 * i + pa];
 #pragma unroll
-        for (int j = 0; j < NC; ++j) yv[j] = sd[kk * kTileAo + wc * hc + 16 * j + l16];
+        for (int j = 0; j < NC; ++j) yv[j] = sd[kk * CW + wc * hc + 16 * j + l16];
 #pragma unroll
         for (int i = 0; i < NR; ++i)
 #pragma unroll
@@ -1940,8 +1962,9 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
       cur = cur + 1 == P::NS ? 0 : cur + 1;
     }
   });
-  den_tile_epilogue<S, GGA, true, STORE>(a, ao, it, L, acc, part,
-                                         reinterpret_cast<double *>(s_stage), s_red, &pre, kq);
+  den_tile_epilogue<S, GGA, true, STORE, CM>(a, ao, it, L, acc, part,
+                                             reinterpret_cast<double *>(s_stage), s_red, &pre,
+                                             kq);
 }
 
 // The density items (STORE = false: restricted, D2 symmetric).  STORE: rho (and
@@ -1951,8 +1974,8 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
 // per-leaf k_density_wave took 5.2, the three tau passes 5.3 ms (4.2e9 bytes
 // of plane each read once for the k-loop and once for the row sums; without
 // SYM's shorter k-loop 20 to 30 % more MFMAs) where it took 12.7.
-template <typename S, bool GGA, bool SYM, bool STORE>
-__global__ __launch_bounds__(256, 2) void k_den_tile_dma(BuildArgs a, const S *__restrict__ ao,
+template <typename S, bool GGA, bool SYM, bool STORE, int CW>
+__global__ __launch_bounds__(256, CW == 64 ? 3 : 2) void k_den_tile_dma(BuildArgs a, const S *__restrict__ ao,
                                                          const int *__restrict__ ao_map,
                                                          const DenItem *__restrict__ items,
                                                          double *__restrict__ part, int plane0) {
@@ -1960,11 +1983,12 @@ __global__ __launch_bounds__(256, 2) void k_den_tile_dma(BuildArgs a, const S *_
   // second __shared__ variable the LDS accesses carry alias scopes, and the
   // compiler then waits for every direct load in flight before each chunk's
   // LDS reads, which serialises the load pipeline
-  __shared__ __align__(16) char s_stage[DenDma<S>::NS * DenDma<S>::STAGE + 4 * sizeof(double)];
-  double *s_red = reinterpret_cast<double *>(s_stage + DenDma<S>::NS * DenDma<S>::STAGE);
+  using P = DenDma<S, CW>;
+  __shared__ __align__(16) char s_stage[P::NS * P::STAGE + 4 * sizeof(double)];
+  double *s_red = reinterpret_cast<double *>(s_stage + P::NS * P::STAGE);
   const DenItem it = items[blockIdx.x];
   if (it.leaf < 0) return;
-  den_tile_item_dma<S, GGA, SYM, STORE>(a, ao, ao_map, it, part, s_stage, s_red,
+  den_tile_item_dma<S, GGA, SYM, STORE, CW>(a, ao, ao_map, it, part, s_stage, s_red,
                                         plane0 + blockIdx.y, blockIdx.y);
 }
 
@@ -2049,8 +2073,9 @@ __global__ __launch_bounds__(256) void k_den_finish_store(BuildArgs a,
 // (k_vxc_gemm_f32: 2.5 ms of 23.8 on (H2O)128 / def2-SVP; k_vxc_dma: 0.3 ms of
 // 3.6 on (H2O)32); in the register-staged ones the atomics drain behind other
 // workgroups' staging and the fold's barriers cost more than it saves.
-template <bool F32, bool FOLD>
-__device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem &it,
+// MT: tiles of a wavefront each way (4, or 2 for blocks of at most 64 AOs).
+template <bool F32, bool FOLD, int MT = 4>
+__device__ __forceinline__ void vxc_scatter(const d4 (&acc)[MT][MT], const VxcItem &it,
                                             const LeafDev &L, const MolDev &MD,
                                             const int *__restrict__ map, double *Km, double cut,
                                             double *s_t) {
@@ -2062,13 +2087,13 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
   auto lrow = [&](int i, int r) { return 16 * i + (F32 ? 4 * g + r : g + 4 * r); };
   if (!FOLD || it.r0 != it.c0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < MT; ++j) {
       if (j >= CT) break;
       const int nu = it.c0 + wcw * hc + 16 * j + l16;
       if (nu >= L.m) continue;
       double *kc = Km + map[nu];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < MT; ++i) {
         if (i >= RT) break;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -2082,17 +2107,17 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
   }
   // K offsets of the entries' rows and columns, loaded once (-1: past the
   // leaf's AOs)
-  long long ro[4][4];
-  int co[4];
+  long long ro[MT][4];
+  int co[MT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int mu = it.r0 + wr * hr + lrow(i, r);
       ro[i][r] = i < RT && mu < L.m ? (long long)map[mu] * MD.nbf : -1;
     }
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < MT; ++j) {
     const int nu = it.c0 + wcw * hc + 16 * j + l16;
     co[j] = j < CT && nu < L.m ? map[nu] : -1;
   }
@@ -2106,13 +2131,13 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
       atomicAdd(Km + ro[i][r] + co[j], v);
   };
   // [row][col ^ (row % 16)] keeps a wavefront's column reads off one bank
-  auto tix = [](int row, int col) { return row * 64 + (col ^ (row & 15)); };
+  auto tix = [](int row, int col) { return row * 16 * MT + (col ^ (row & 15)); };
   auto put = [&](double *T) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < MT; ++i) {
       if (i >= RT) break;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         if (j >= CT) break;
 #pragma unroll
         for (int r = 0; r < 4; ++r) T[tix(lrow(i, r), 16 * j + l16)] = acc[i][j][r];
@@ -2122,10 +2147,10 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
   // upper triangle of a diagonal quadrant from its own transpose T
   auto fold_diag = [&](const double *T) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < MT; ++i) {
       if (i >= RT) break;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         if (j >= CT) break;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -2136,7 +2161,7 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
       }
     }
   };
-  double *R0 = s_t, *R1 = s_t + 64 * 64;
+  double *R0 = s_t, *R1 = s_t + 256 * MT * MT;
   __syncthreads();  // every wavefront is done with the chunk buffers
   if (wave == 1) put(R0);
   if (wave == 0) {
@@ -2147,10 +2172,10 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[4][4], const VxcItem
   if (wave == 2) {
     // upper-right quadrant entry (lr, lc) + lower-left entry (lc, lr)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < MT; ++i) {
       if (i >= RT) break;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         if (j >= CT) break;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -2529,20 +2554,26 @@ __global__ __launch_bounds__(256, 2) void k_vxc_gemm_f32(BuildArgs a, const floa
 // form 6.46 ms (2.9 times the MFMAs; its scatter drops nothing above 1e-18).  A chunk's operands fill the registers (128 of the 256
 // hold accumulators): Phi is read last, and TAU keeps its plane loop rolled,
 // without which 18 and 40 of them spill.
-constexpr int kVdRow = 64;                         // bytes of a row in a chunk
-constexpr int kVdPlane = 2 * kTileAo * kVdRow;     // bytes of one plane's rows
+// MT = 2: a context whose blocks are all at most 64 AOs wide; half the LDS and
+// a quarter of the accumulators, so that four workgroups share a CU.
+constexpr int kVdRow = 64;                                        // bytes of a row in a chunk
+template <int MT> constexpr int vd_plane() { return 64 * MT * kVdRow; }  // one plane's rows
 template <typename S> constexpr int vd_pts() { return kVdRow / (int)sizeof(S); }
-// coefficients of a chunk behind the planes: [planes][points] doubles
-template <typename S, bool GGA, bool TAU> constexpr int vd_smem() {
-  return (GGA ? 4 : 1) * kVdPlane + (GGA ? 4 + (TAU ? 1 : 0) : 1) * vd_pts<S>() * 8;
+// coefficients of a chunk behind the planes: [planes][points] doubles; at least
+// the scatter's transposes
+template <typename S, bool GGA, bool TAU, int MT> constexpr int vd_smem() {
+  const int stage = (GGA ? 4 : 1) * vd_plane<MT>() + (GGA ? 4 + (TAU ? 1 : 0) : 1) * vd_pts<S>() * 8;
+  const int trans = 2 * 256 * MT * MT * 8;
+  return stage > trans ? stage : trans;
 }
 
-template <typename S, bool GGA, bool TAU>
+template <typename S, bool GGA, bool TAU, int MT>
 __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__restrict__ ao,
                                              const int *__restrict__ ao_map, const VxcItem &it,
                                              char *s_stage) {
   static_assert(GGA || !TAU, "tau terms come with the GGA planes");
   constexpr int PT = vd_pts<S>(), NQ = GGA ? 4 : 1, NC = NQ + (TAU ? 1 : 0);
+  constexpr int PL = vd_plane<MT>();
   constexpr int NH = PT / 8;  // operand rounds of 8 points per chunk
   const LeafDev L = a.leaves[it.leaf];
   const MolDev MD = a.mols[L.mol];
@@ -2572,27 +2603,27 @@ __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__rest
   auto dma = [&](int p0) __attribute__((always_inline)) {
     const int q0 = GGA ? wave : 0;
     const S *src = phi + q0 * cs + loff + p0;
-    char *dst = s_stage + q0 * kVdPlane;
+    char *dst = s_stage + q0 * PL;
     for (int k = GGA ? 0 : wave; k < gr + gc; k += GGA ? 1 : 4) {
       const int lr = k < gr ? 16 * k : cb + 16 * (k - gr);
       const int ar = k < gr ? it.r0 + 16 * k : it.c0 + 16 * (k - gr);
       __builtin_amdgcn_global_load_lds(src + (long long)ar * L.np, dst + lr * kVdRow, 16, 0, 0);
     }
     if (wave == 0 && lane < NC * (PT / 2))
-      __builtin_amdgcn_global_load_lds(cptr + p0, s_stage + NQ * kVdPlane, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(cptr + p0, s_stage + NQ * PL, 16, 0, 0);
   };
   const int nch = (L.n + PT - 1) / PT;
   const int RTl = live_tiles(L.m - (it.r0 + wr * hr), hr), CTl = live_tiles(L.m - (it.c0 + wcw * hc), hc);
   if (nch > 0) dma(0);
-  d4 acc[4][4];
+  d4 acc[MT][MT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int j = 0; j < MT; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   // this lane's operand bytes of row tile 0 / column tile 0 in plane 0
   const char *xr = s_stage + (wr * hr + l16) * kVdRow + ((g ^ vxc_swz(l16)) << 4);
   const char *xc = s_stage + (cb + wcw * hc + l16) * kVdRow + ((g ^ vxc_swz(l16)) << 4);
-  const double *sc = reinterpret_cast<const double *>(s_stage + NQ * kVdPlane) + (PT / 4) * g;
+  const double *sc = reinterpret_cast<const double *>(s_stage + NQ * PL) + (PT / 4) * g;
   auto ld = [](const char *p, int h) __attribute__((always_inline)) -> d2u {
     if constexpr (sizeof(S) == 8) {
       return *reinterpret_cast<const d2u *>(p);
@@ -2602,7 +2633,7 @@ __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__rest
       return d2u{(double)v[0], (double)v[1]};
     }
   };
-  tile_shape_ext(RTl, CTl, [&](auto R, auto C) __attribute__((always_inline)) {
+  tile_shape_max<MT, MT>(RTl, CTl, [&](auto R, auto C) __attribute__((always_inline)) {
     constexpr int NR = decltype(R)::value, NCt = decltype(C)::value;
     constexpr int NRs = NR ? NR : 1, NCs = NCt ? NCt : 1;
     for (int c = 0; c < nch; ++c) {
@@ -2633,13 +2664,13 @@ __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__rest
             d2u xk[NRs], yk[NCs];
 #pragma unroll
             for (int j = 0; j < NCt; ++j) {
-              yk[j] = ld(xc + k * kVdPlane + 16 * j * kVdRow, h);
+              yk[j] = ld(xc + k * PL + 16 * j * kVdRow, h);
               ac[j] += ck * yk[j];
             }
             if (TAU || !diag) {
 #pragma unroll
               for (int i = 0; i < NR; ++i) {
-                xk[i] = ld(xr + k * kVdPlane + 16 * i * kVdRow, h);
+                xk[i] = ld(xr + k * PL + 16 * i * kVdRow, h);
                 ar[i] += ck * xk[i];
               }
             }
@@ -2694,17 +2725,17 @@ __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__rest
       }
     }
   });
-  vxc_scatter<false, GGA>(acc, it, L, MD, map, Km, TAU ? kStorageCut : kScatterCut, reinterpret_cast<double*>(s_stage));
+  vxc_scatter<false, true, MT>(acc, it, L, MD, map, Km, TAU ? kStorageCut : kScatterCut, reinterpret_cast<double *>(s_stage));
 }
 
-template <typename S, bool GGA, bool TAU>
-__global__ __launch_bounds__(256, 2) void k_vxc_dma(BuildArgs a, const S *__restrict__ ao,
+template <typename S, bool GGA, bool TAU, int MT>
+__global__ __launch_bounds__(256, MT == 4 ? 2 : TAU ? 3 : 4) void k_vxc_dma(BuildArgs a, const S *__restrict__ ao,
                                                     const int *__restrict__ ao_map,
                                                     const VxcItem *__restrict__ items) {
-  __shared__ __align__(16) char s_stage[vd_smem<S, GGA, TAU>()];
+  __shared__ __align__(16) char s_stage[vd_smem<S, GGA, TAU, MT>()];
   const VxcItem it = items[blockIdx.x];
   if (it.leaf < 0 || !a.leaf_active[it.leaf]) return;
-  vxc_item_dma<S, GGA, TAU>(a, ao, ao_map, it, s_stage);
+  vxc_item_dma<S, GGA, TAU, MT>(a, ao, ao_map, it, s_stage);
 }
 
 // Persistent, wavefront-specialised form of the Vxc items: one 512-thread
@@ -2987,6 +3018,7 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
                            bool vxc_only = false) {
   constexpr int kXcd = kXcdRuns;
   const int nl = (int)leaves.size();
+  p.narrow = true;
   double total = 0.0;
   for (const auto &L : leaves) total += (double)L.np * L.mp * L.mp;
   std::vector<std::vector<DenItem>> den(kXcd);
@@ -2999,6 +3031,7 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
     const int x = std::min(kXcd - 1, (int)(acc / std::max(total, 1.0) * kXcd));
     acc += (double)L.np * L.mp * L.mp;
     const auto cb = tile_blocks(L.mp, p.tune.tile_ao);
+    if (cb[0].second > 64) p.narrow = false;  // the first block is the widest
     std::vector<std::pair<int, int>> pb;
     for (int p0 = 0; p0 < L.np; p0 += kTileAo) pb.push_back({p0, std::min(kTileAo, L.np - p0)});
     const bool single = cb.size() == 1 && pb.size() == 1;
@@ -3150,7 +3183,10 @@ void run_density_store(const ContractPlan &plan, const BuildArgs &a, const void 
       using S = decltype(s_tag);
       BuildArgs x = a;
       x.D2 = D2t;
-      (a.deriv ? k_den_tile_dma<S, true, false, true> : k_den_tile_dma<S, false, false, true>)
+      (plan.narrow ? (a.deriv ? k_den_tile_dma<S, true, false, true, 64>
+                              : k_den_tile_dma<S, false, false, true, 64>)
+                   : (a.deriv ? k_den_tile_dma<S, true, false, true, 128>
+                              : k_den_tile_dma<S, false, false, true, 128>))
           <<<plan.n_den_items, 256, 0, s>>>(x, static_cast<const S *>(ao), a.ao_map,
                                             plan.den_items.get(), plan.den_part.get(), 0);
     };
@@ -3181,7 +3217,8 @@ void run_tau_store(const ContractPlan &plan, const BuildArgs &a, const LeafDev *
       using S = decltype(s_tag);
       BuildArgs x = a;
       x.D2 = D2s;
-      k_den_tile_dma<S, false, true, true><<<dim3(plan.n_den_items, 3), 256, 0, s>>>(
+      (plan.narrow ? k_den_tile_dma<S, false, true, true, 64>
+                   : k_den_tile_dma<S, false, true, true, 128>)<<<dim3(plan.n_den_items, 3), 256, 0, s>>>(
           x, static_cast<const S *>(ao), a.ao_map, plan.den_items.get(), plan.den_part.get(), 1);
     };
     if (precision == 0) launch(double{});
@@ -3216,7 +3253,10 @@ void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, i
             <<<std::min(2 * plan.persistent_wgs, plan.n_den_items), 256, 0, s>>>(
                 a, x, plan.den_items.get(), plan.den_part.get(), plan.n_den_items);
       else if (plan.den_dma)
-        (a.deriv ? k_den_tile_dma<S, true, false, false> : k_den_tile_dma<S, false, true, false>)
+        (plan.narrow ? (a.deriv ? k_den_tile_dma<S, true, false, false, 64>
+                                : k_den_tile_dma<S, false, true, false, 64>)
+                     : (a.deriv ? k_den_tile_dma<S, true, false, false, 128>
+                                : k_den_tile_dma<S, false, true, false, 128>))
             <<<plan.n_den_items, 256, 0, s>>>(a, x, a.ao_map, plan.den_items.get(),
                                               plan.den_part.get(), 0);
       else
@@ -3375,7 +3415,8 @@ void run_vxc(const ContractPlan &plan, const BuildArgs &a, const void *ao, int p
         check_launch("k_vxc_ws");
         return;
       }
-      (a.deriv ? k_vxc_dma<S, true, false> : k_vxc_dma<S, false, false>)
+      (plan.narrow ? (a.deriv ? k_vxc_dma<S, true, false, 2> : k_vxc_dma<S, false, false, 2>)
+                   : (a.deriv ? k_vxc_dma<S, true, false, 4> : k_vxc_dma<S, false, false, 4>))
           <<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const S *>(ao), a.ao_map,
                                             plan.vxc_items.get());
       check_launch("k_vxc_dma");
@@ -3426,12 +3467,14 @@ void run_vxc_mgga(const ContractPlan &plan, const BuildArgs &a, const LeafDev *l
   if (a.nleaves == 0) return;
   if (plan.tiled) {
     // the GGA term and the three tau terms of a block pair in one item
-    if (precision == 0)
-      k_vxc_dma<double, true, true><<<plan.n_vxc_items, 256, 0, s>>>(
-          a, static_cast<const double *>(ao), a.ao_map, plan.vxc_items.get());
-    else
-      k_vxc_dma<float, true, true><<<plan.n_vxc_items, 256, 0, s>>>(
-          a, static_cast<const float *>(ao), a.ao_map, plan.vxc_items.get());
+    auto launch = [&](auto s_tag) {
+      using S = decltype(s_tag);
+      (plan.narrow ? k_vxc_dma<S, true, true, 2> : k_vxc_dma<S, true, true, 4>)
+          <<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const S *>(ao), a.ao_map,
+                                            plan.vxc_items.get());
+    };
+    if (precision == 0) launch(double{});
+    else launch(float{});
     check_launch("k_vxc_dma (meta-GGA)");
     return;
   }
