@@ -1611,6 +1611,29 @@ __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *_
   const S *phi = ao + L.ao_off;
   const long long cs = (long long)L.mp * L.np;
   __syncthreads();  // s_phi is reused for the sums below
+  // rounds of NJ column tiles' loads, kept as stored; with two column tiles the
+  // next round's loads are issued before this round's are used (with four there
+  // are no registers for them)
+  using V = typename Vec4Of<S>::type;
+  using First = DenEpiFirst<S, CM>;
+  constexpr int NJ = First::NJ;
+  auto load = [&](int i, int jj, First &d) __attribute__((always_inline)) {
+    const int pl = wp * hp + 16 * i + 4 * g;
+#pragma unroll
+    for (int jq = 0; jq < NJ; ++jq) {
+      if (jj + jq >= CT) break;
+      const long long off = (long long)(it.c0 + wc * hc + 16 * (jj + jq) + l16) * L.np + it.p0 + pl;
+      d.f[jq] = *reinterpret_cast<const V *>(phi + off);
+      if constexpr (GGA) {
+        d.fx[jq] = *reinterpret_cast<const V *>(phi + cs + off);
+        d.fy[jq] = *reinterpret_cast<const V *>(phi + 2 * cs + off);
+        d.fz[jq] = *reinterpret_cast<const V *>(phi + 3 * cs + off);
+      }
+    }
+  };
+  constexpr bool kAhead = PRE && CM == 2;
+  First cur, nxt;
+  if constexpr (kAhead) cur = *pre;
   // acc[i][j][r] = T(point wp*hp + 16 i + 4 g + r, column wc*hc + 16 j + l16)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -1621,49 +1644,29 @@ __device__ __forceinline__ void den_tile_epilogue(const BuildArgs &a, const S *_
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int k = 0; k < 4; ++k) q[r][k] = 0.0;
-    // NJ column tiles' loads in flight before any is used, kept as stored
-    // (64 registers of loads: all four tiles with FP32 storage, two with FP64)
-    using V = typename Vec4Of<S>::type;
-    constexpr int NJ = DenEpiFirst<S, CM>::NJ;
 #pragma unroll
     for (int jj = 0; jj < CM; jj += NJ) {
-      V f[NJ], fx[NJ], fy[NJ], fz[NJ];
-#pragma unroll
-      for (int jq = 0; jq < NJ; ++jq) {
-        if (jj + jq >= CT) break;
-        if (PRE && i == 0 && jj == 0) {
-          f[jq] = pre->f[jq];
-          if constexpr (GGA) {
-            fx[jq] = pre->fx[jq];
-            fy[jq] = pre->fy[jq];
-            fz[jq] = pre->fz[jq];
-          }
-          continue;
-        }
-        const long long off = (long long)(it.c0 + wc * hc + 16 * (jj + jq) + l16) * L.np + it.p0 + pl;
-        f[jq] = *reinterpret_cast<const V *>(phi + off);
-        if constexpr (GGA) {
-          fx[jq] = *reinterpret_cast<const V *>(phi + cs + off);
-          fy[jq] = *reinterpret_cast<const V *>(phi + 2 * cs + off);
-          fz[jq] = *reinterpret_cast<const V *>(phi + 3 * cs + off);
-        }
-      }
+      if (jj >= CT) break;
+      if constexpr (!kAhead) load(i, jj, cur);
+      else if (jj + NJ < CM && jj + NJ < CT) load(i, jj + NJ, nxt);
+      else if (i + 1 < 4 && i + 1 < RT) load(i + 1, 0, nxt);
 #pragma unroll
       for (int jq = 0; jq < NJ; ++jq) {
         const int j = jj + jq;
         if (j >= CT) break;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) q[r][0] += (double)f[jq][r] * acc[i][j][r];
+        for (int r = 0; r < 4; ++r) q[r][0] += (double)cur.f[jq][r] * acc[i][j][r];
         if constexpr (GGA) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const double tt = 2.0 * acc[i][j][r];
-            q[r][1] += (double)fx[jq][r] * tt;
-            q[r][2] += (double)fy[jq][r] * tt;
-            q[r][3] += (double)fz[jq][r] * tt;
+            q[r][1] += (double)cur.fx[jq][r] * tt;
+            q[r][2] += (double)cur.fy[jq][r] * tt;
+            q[r][3] += (double)cur.fz[jq][r] * tt;
           }
         }
       }
+      if constexpr (kAhead) cur = nxt;
     }
     // the column sums: lane l16 of a row ends with point pl + l16 / 4's
     // quantity l16 % 4 (GGA) or point pl + l16 / 4's rho (LDA)
@@ -1817,18 +1820,21 @@ __device__ __forceinline__ void den_tile_item(const BuildArgs &a, const S *__res
 // the unused tiles read), so a chunk's loads are waited for by count.  The
 // MFMA k-step t reads AO 4 g + t of both, so the accumulators are those of
 // den_tile_item and the epilogue is shared.
-// CW: the widest column block, 128 or, where a context's blocks are all at most
-// 64 AOs wide (small molecules), 64: half the accumulators and 24 KB (FP64)
-// buffers, so that three workgroups share a CU instead of two and the few
-// hundred items of a small molecule run in one round (water / 6-31G: 23.9 ->
-// 17.4 us; the Vxc items, four to a CU, 16.4 -> 12.8 us).
-template <typename S, int CW = kTileAo> struct DenDma {
+// Column blocks are at most kDenAo = 64 AOs wide: with 128 the accumulators and
+// buffers let two workgroups share a CU, with 64 three, which hide more of each
+// other's epilogue loads and give a small molecule's items one round.  Density
+// stage, 128 -> 64 wide: (H2O)32 PBE FP64 3.05 -> 2.96 ms, TPSS 9.1 -> 8.5,
+// C30H62 BLYP FP32 storage 2.37 -> 2.18, (H2O)128 20.0 -> 19.35, water 23.9 ->
+// 17.4 us, though Phi is read once per 64 columns.
+constexpr int kDenAo = 64;
+template <typename S> struct DenDma {
+  static constexpr int CW = kDenAo;
   static constexpr int NS = sizeof(S) == 8 ? 2 : 3;               // LDS chunk buffers
   static constexpr int PHI = kTKc * kTileAo * (int)sizeof(S);     // bytes of Phi per buffer
   static constexpr int STAGE = PHI + kTKc * CW * 8;               // bytes per buffer
   static constexpr int LOADS = (sizeof(S) == 8 ? 4 : 2) + CW / 8; // loads per chunk per wavefront
 };
-static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float, 64>::STAGE / 8, "epilogue sums fit a stage");
+static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float>::STAGE / 8, "epilogue sums fit a stage");
 
 // SYM (LDA form, symmetric D2): only the row sums of (Phi D2) o Phi are
 // wanted, so the k-loop of column block [c0, c0 + wc) stops at the block's end
@@ -1836,15 +1842,15 @@ static_assert(4 * kMaxLeafPts + 4 * kTileAo <= DenDma<float, 64>::STAGE / 8, "ep
 // the loads of a leaf of nb blocks go.
 // plane: the AO plane in Phi's place (1..3: the meta-GGA's tau passes, LDA
 // form), its sums going to quantity kq of the stored planes.
-template <typename S, bool GGA, bool SYM, bool STORE, int CW>
+template <typename S, bool GGA, bool SYM, bool STORE>
 __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *__restrict__ ao,
                                                   const int *__restrict__ ao_map,
                                                   const DenItem &it, double *__restrict__ part,
                                                   char *s_stage, double *s_red, int plane = 0,
                                                   int kq = 0) {
   static_assert(!(GGA && SYM), "grad rho needs all of Phi D2");
-  using P = DenDma<S, CW>;
-  constexpr int CM = CW / 32;  // column tiles of a wavefront
+  using P = DenDma<S>;
+  constexpr int CW = P::CW, CM = CW / 32;  // column tiles of a wavefront
   LeafDev L = a.leaves[it.leaf];
   if constexpr (STORE && !GGA) L.ao_off += (long long)plane * L.mp * L.np;
   const MolDev MD = a.mols[L.mol];
@@ -1974,8 +1980,8 @@ __device__ __forceinline__ void den_tile_item_dma(const BuildArgs &a, const S *_
 // per-leaf k_density_wave took 5.2, the three tau passes 5.3 ms (4.2e9 bytes
 // of plane each read once for the k-loop and once for the row sums; without
 // SYM's shorter k-loop 20 to 30 % more MFMAs) where it took 12.7.
-template <typename S, bool GGA, bool SYM, bool STORE, int CW>
-__global__ __launch_bounds__(256, CW == 64 ? 3 : 2) void k_den_tile_dma(BuildArgs a, const S *__restrict__ ao,
+template <typename S, bool GGA, bool SYM, bool STORE>
+__global__ __launch_bounds__(256, 3) void k_den_tile_dma(BuildArgs a, const S *__restrict__ ao,
                                                          const int *__restrict__ ao_map,
                                                          const DenItem *__restrict__ items,
                                                          double *__restrict__ part, int plane0) {
@@ -1983,12 +1989,12 @@ __global__ __launch_bounds__(256, CW == 64 ? 3 : 2) void k_den_tile_dma(BuildArg
   // second __shared__ variable the LDS accesses carry alias scopes, and the
   // compiler then waits for every direct load in flight before each chunk's
   // LDS reads, which serialises the load pipeline
-  using P = DenDma<S, CW>;
+  using P = DenDma<S>;
   __shared__ __align__(16) char s_stage[P::NS * P::STAGE + 4 * sizeof(double)];
   double *s_red = reinterpret_cast<double *>(s_stage + P::NS * P::STAGE);
   const DenItem it = items[blockIdx.x];
   if (it.leaf < 0) return;
-  den_tile_item_dma<S, GGA, SYM, STORE, CW>(a, ao, ao_map, it, part, s_stage, s_red,
+  den_tile_item_dma<S, GGA, SYM, STORE>(a, ao, ao_map, it, part, s_stage, s_red,
                                         plane0 + blockIdx.y, blockIdx.y);
 }
 
@@ -2949,7 +2955,7 @@ static std::vector<std::pair<int, int>> tile_blocks(int n, int maxw = kTileAo) {
 }
 
 double tile_plan_bytes(const LeafDev &L) {
-  const double ncb = (double)tile_blocks(L.mp).size();
+  const double ncb = (double)tile_blocks(L.mp, kDenAo).size();
   const double npb = (double)((L.np + kTileAo - 1) / kTileAo);
   const double parts = ncb * npb > 1.0 ? ncb * npb : 0.0;
   return parts * 4 * kTileAo * sizeof(double) + ncb * npb * sizeof(DenItem) +
@@ -3019,6 +3025,8 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
   constexpr int kXcd = kXcdRuns;
   const int nl = (int)leaves.size();
   p.narrow = true;
+  // the directly loaded density items are at most kDenAo wide
+  const int den_ao = p.den_dma && !p.den_persistent ? std::min(p.tune.tile_ao, kDenAo) : p.tune.tile_ao;
   double total = 0.0;
   for (const auto &L : leaves) total += (double)L.np * L.mp * L.mp;
   std::vector<std::vector<DenItem>> den(kXcd);
@@ -3034,14 +3042,15 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
     if (cb[0].second > 64) p.narrow = false;  // the first block is the widest
     std::vector<std::pair<int, int>> pb;
     for (int p0 = 0; p0 < L.np; p0 += kTileAo) pb.push_back({p0, std::min(kTileAo, L.np - p0)});
-    const bool single = cb.size() == 1 && pb.size() == 1;
-    if (!single) fin.push_back(DenFinish{li, nparts, (int)cb.size(), (int)pb.size()});
+    const auto db = tile_blocks(L.mp, den_ao);
+    const bool single = db.size() == 1 && pb.size() == 1;
+    if (!single) fin.push_back(DenFinish{li, nparts, (int)db.size(), (int)pb.size()});
     for (size_t ip = 0; ip < pb.size(); ++ip)
-      for (size_t ic = 0; ic < cb.size(); ++ic)
-        den[x].push_back(DenItem{li, single ? -1 : nparts + (int)(ip * cb.size() + ic),
+      for (size_t ic = 0; ic < db.size(); ++ic)
+        den[x].push_back(DenItem{li, single ? -1 : nparts + (int)(ip * db.size() + ic),
                                  (short)pb[ip].first, (short)pb[ip].second,
-                                 (short)cb[ic].first, (short)cb[ic].second});
-    if (!single) nparts += (int)(cb.size() * pb.size());
+                                 (short)db[ic].first, (short)db[ic].second});
+    if (!single) nparts += (int)(db.size() * pb.size());
     for (size_t r = 0; r < cb.size(); ++r)
       for (size_t c = r; c < cb.size(); ++c)
         vxc[x].push_back(VxcItem{li, (short)cb[r].first, (short)cb[r].second,
@@ -3108,15 +3117,15 @@ ContractPlan make_contract_plan(const std::vector<LeafDev> &leaves, long long mt
   p.two_pass = p.vxc_variant == 2 && precision != 2;  // not with the split-BF16 Vxc
   p.tiled = tiled_setting(precision);
   if (p.tiled) {
+    p.vxc_ws = (p.tune.persistent & 2) != 0;
+    p.den_persistent = (p.tune.persistent & 1) != 0;
+    const char *dd = std::getenv("OCCXC_DENSITY_DMA");
+    p.den_dma = dd ? std::atoi(dd) != 0 : kDefaultDensityDma;
     make_tile_plan(p, leaves);
     int dev = 0, cus = 0;
     OCCXC_HIP(hipGetDevice(&dev));
     OCCXC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     p.persistent_wgs = std::max(8, cus / 8 * 8);
-    p.vxc_ws = (p.tune.persistent & 2) != 0;
-    p.den_persistent = (p.tune.persistent & 1) != 0;
-    const char *dd = std::getenv("OCCXC_DENSITY_DMA");
-    p.den_dma = dd ? std::atoi(dd) != 0 : kDefaultDensityDma;
     for (const void *k : {reinterpret_cast<const void *>(&k_vxc_ws<double, true>),
                           reinterpret_cast<const void *>(&k_vxc_ws<double, false>),
                           reinterpret_cast<const void *>(&k_vxc_ws<float, true>),
@@ -3178,15 +3187,12 @@ ContractPlan make_contract_plan(const std::vector<LeafDev> &leaves, long long mt
 void run_density_store(const ContractPlan &plan, const BuildArgs &a, const void *ao,
                        int precision, const double *D2t, hipStream_t s) {
   if (a.nleaves == 0) return;
-  if (plan.tiled && plan.den_dma) {
+  if (plan.tiled && plan.den_dma && !plan.den_persistent) {
     auto launch = [&](auto s_tag) {
       using S = decltype(s_tag);
       BuildArgs x = a;
       x.D2 = D2t;
-      (plan.narrow ? (a.deriv ? k_den_tile_dma<S, true, false, true, 64>
-                              : k_den_tile_dma<S, false, false, true, 64>)
-                   : (a.deriv ? k_den_tile_dma<S, true, false, true, 128>
-                              : k_den_tile_dma<S, false, false, true, 128>))
+      (a.deriv ? k_den_tile_dma<S, true, false, true> : k_den_tile_dma<S, false, false, true>)
           <<<plan.n_den_items, 256, 0, s>>>(x, static_cast<const S *>(ao), a.ao_map,
                                             plan.den_items.get(), plan.den_part.get(), 0);
     };
@@ -3212,13 +3218,12 @@ void run_density_store(const ContractPlan &plan, const BuildArgs &a, const void 
 void run_tau_store(const ContractPlan &plan, const BuildArgs &a, const LeafDev *leaves_k,
                    const void *ao, int precision, const double *D2s, hipStream_t s) {
   if (a.nleaves == 0) return;
-  if (plan.tiled && plan.den_dma) {
+  if (plan.tiled && plan.den_dma && !plan.den_persistent) {
     auto launch = [&](auto s_tag) {
       using S = decltype(s_tag);
       BuildArgs x = a;
       x.D2 = D2s;
-      (plan.narrow ? k_den_tile_dma<S, false, true, true, 64>
-                   : k_den_tile_dma<S, false, true, true, 128>)<<<dim3(plan.n_den_items, 3), 256, 0, s>>>(
+      k_den_tile_dma<S, false, true, true><<<dim3(plan.n_den_items, 3), 256, 0, s>>>(
           x, static_cast<const S *>(ao), a.ao_map, plan.den_items.get(), plan.den_part.get(), 1);
     };
     if (precision == 0) launch(double{});
@@ -3253,10 +3258,7 @@ void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, i
             <<<std::min(2 * plan.persistent_wgs, plan.n_den_items), 256, 0, s>>>(
                 a, x, plan.den_items.get(), plan.den_part.get(), plan.n_den_items);
       else if (plan.den_dma)
-        (plan.narrow ? (a.deriv ? k_den_tile_dma<S, true, false, false, 64>
-                                : k_den_tile_dma<S, false, true, false, 64>)
-                     : (a.deriv ? k_den_tile_dma<S, true, false, false, 128>
-                                : k_den_tile_dma<S, false, true, false, 128>))
+        (a.deriv ? k_den_tile_dma<S, true, false, false> : k_den_tile_dma<S, false, true, false>)
             <<<plan.n_den_items, 256, 0, s>>>(a, x, a.ao_map, plan.den_items.get(),
                                               plan.den_part.get(), 0);
       else

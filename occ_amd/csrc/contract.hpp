@@ -41,7 +41,7 @@ struct ContractPlan {
   bool vxc_ws = false;     // persistent wavefront-specialised Vxc instead of one item per workgroup
   bool den_persistent = false;  // persistent density launch (workgroups loop over items)
   bool den_dma = false;   // density items staged by direct-to-LDS loads (k_den_tile_dma)
-  bool narrow = false;    // every AO block is at most 64 wide: the kernels' narrow forms
+  bool narrow = false;    // every Vxc AO block is at most 64 wide: the kernel's narrow form
   int persistent_wgs = 256;  // workgroups of the persistent kernels (a multiple of 8)
   int n_den_items = 0, n_vxc_items = 0, n_den_finish = 0, n_den_parts = 0;
   DevBuf<DenItem> den_items;
