@@ -1003,28 +1003,36 @@ __global__ __launch_bounds__(256) void k_eval_basis_flat(const ShellDev *__restr
   }
 }
 
-__global__ void k_decay_cutoff(const ShellDev *__restrict__ shells, int nshell,
-                               const double *__restrict__ exps,
-                               const double *__restrict__ coefs, double thr,
-                               double *__restrict__ ext) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nshell) return;
-  const ShellDev sh = shells[s];
+__global__ __launch_bounds__(64) void k_decay_cutoff(const ShellDev *__restrict__ shells,
+                                                     int nshell, const double *__restrict__ exps,
+                                                     const double *__restrict__ coefs, double thr,
+                                                     double *__restrict__ ext) {
+  const ShellDev sh = shells[blockIdx.x];
   const double max_radius = 30.0, increment = 0.1, min_radius = 0.5;
   const int npts = (int)((max_radius - min_radius) / increment) + 1;
   const double step = (max_radius - min_radius) / (double)(npts - 1);
-  double result = 0.0;
-  for (int i = 0; i < npts; ++i) {
-    const double r = (i == npts - 1) ? max_radius : min_radius + (double)i * step;
-    const double x = 1.0 * r + sh.x, y = 0.0 + sh.y, z = 0.0 + sh.z;
-    double o[4][kNCartMax];
-    eval_shell(sh, exps, coefs, x - sh.x, y - sh.y, z - sh.z, false, o);
-    result = i * increment + min_radius;
-    double v = 0.0;
-    for (int c = 0; c < sh.size; ++c) v = fmax(v, fabs(o[0][c]));
-    if (v < thr) break;
+  // 64 radii at a time, the first one below the threshold ends the scan (one
+  // thread per shell took the 296 radii one after the other: 206 us)
+  int stop = npts - 1;
+  for (int i0 = 0; i0 < npts; i0 += 64) {
+    const int i = i0 + threadIdx.x;
+    bool below = false;
+    if (i < npts) {
+      const double r = (i == npts - 1) ? max_radius : min_radius + (double)i * step;
+      const double x = 1.0 * r + sh.x, y = 0.0 + sh.y, z = 0.0 + sh.z;
+      double o[4][kNCartMax];
+      eval_shell(sh, exps, coefs, x - sh.x, y - sh.y, z - sh.z, false, o);
+      double v = 0.0;
+      for (int c = 0; c < sh.size; ++c) v = fmax(v, fabs(o[0][c]));
+      below = v < thr;
+    }
+    const unsigned long long hit = __ballot(below);
+    if (hit) {
+      stop = i0 + __ffsll(hit) - 1;
+      break;
+    }
   }
-  ext[s] = result;
+  if (threadIdx.x == 0) ext[blockIdx.x] = stop * increment + min_radius;
 }
 
 __global__ void k_functional(int id, long long n, const double *__restrict__ rho,
@@ -1341,8 +1349,7 @@ void launch_decay_cutoff(const ShellDev *shells, int nshell, const double *exps,
                          const double *coefs, double threshold, double *extents,
                          hipStream_t s) {
   if (nshell == 0) return;
-  k_decay_cutoff<<<grid_for(nshell, 64), 64, 0, s>>>(shells, nshell, exps, coefs, threshold,
-                                                     extents);
+  k_decay_cutoff<<<nshell, 64, 0, s>>>(shells, nshell, exps, coefs, threshold, extents);
   check_launch();
 }
 

@@ -62,15 +62,23 @@ __global__ __launch_bounds__(256) void k_bbox_part(const double *__restrict__ xy
   if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
 }
 
-// box = {min x, min y, min z, extent x, y, z}; an extent below 1e-10 becomes 1
-__global__ void k_bbox_final(const double *__restrict__ part, int nb, double *__restrict__ box) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// box = {min x, min y, min z, extent x, y, z}; an extent below 1e-10 becomes 1.
+// One wavefront: lanes take every 64th part (one thread over all parts waited
+// for each of their loads, 56 us).
+__global__ __launch_bounds__(64) void k_bbox_final(const double *__restrict__ part, int nb,
+                                                   double *__restrict__ box) {
   double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-  for (int b = 0; b < nb; ++b)
+  for (int b = threadIdx.x; b < nb; b += 64)
     for (int k = 0; k < 3; ++k) {
       mn[k] = fmin(mn[k], part[6 * b + k]);
       mx[k] = fmax(mx[k], part[6 * b + 3 + k]);
     }
+  for (int w = 32; w > 0; w >>= 1)
+    for (int k = 0; k < 3; ++k) {
+      mn[k] = fmin(mn[k], __shfl_xor(mn[k], w, 64));
+      mx[k] = fmax(mx[k], __shfl_xor(mx[k], w, 64));
+    }
+  if (threadIdx.x != 0) return;
   for (int k = 0; k < 3; ++k) {
     double e = mx[k] - mn[k];
     if (e < 1e-10) e = 1.0;
@@ -100,30 +108,39 @@ __device__ __forceinline__ long long leaf_count(long long n, int nleaves, int li
   return li < nleaves - 1 ? kLeafTarget : n - (long long)kLeafTarget * li;
 }
 
-// One thread per leaf: centroid summed in point order, then the largest
-// distance to it (no fused multiply-adds, as on the host).
-__global__ __launch_bounds__(256) void k_leaf_geom(const double *__restrict__ xyz,
-                                                   const int *__restrict__ perm, long long n,
-                                                   int nleaves, double *__restrict__ center,
-                                                   double *__restrict__ radius) {
+// One wavefront per leaf: the leaf's points to LDS, the centroid summed in
+// point order by one lane per axis (no fused multiply-adds, as on the host),
+// then the largest distance to it over the lanes (a maximum does not depend on
+// the order).  One thread per leaf waited for its gathers one by one: 129 us for
+// 1140 leaves.
+__global__ __launch_bounds__(64) void k_leaf_geom(const double *__restrict__ xyz,
+                                                  const int *__restrict__ perm, long long n,
+                                                  int nleaves, double *__restrict__ center,
+                                                  double *__restrict__ radius) {
 #pragma clang fp contract(off)
-  const int li = blockIdx.x * 256 + threadIdx.x;
-  if (li >= nleaves) return;
-  const long long off = (long long)kLeafTarget * li, cnt = leaf_count(n, nleaves, li);
-  double c[3] = {0.0, 0.0, 0.0};
-  for (long long i = 0; i < cnt; ++i) {
+  __shared__ double s_p[3][kMaxLeafPts], s_c[3];
+  const int li = blockIdx.x, lane = threadIdx.x;
+  const long long off = (long long)kLeafTarget * li;
+  const int cnt = (int)leaf_count(n, nleaves, li);
+  for (int i = lane; i < cnt; i += 64) {
     const long long o = perm[off + i];
-    for (int k = 0; k < 3; ++k) c[k] += xyz[3 * o + k];
+    for (int k = 0; k < 3; ++k) s_p[k][i] = xyz[3 * o + k];
   }
-  for (int k = 0; k < 3; ++k) c[k] /= (double)cnt;
+  __syncthreads();
+  if (lane < 3) {
+    double c = 0.0;
+    for (int i = 0; i < cnt; ++i) c += s_p[lane][i];
+    s_c[lane] = c / (double)cnt;
+  }
+  __syncthreads();
   double r = 0.0;
-  for (long long i = 0; i < cnt; ++i) {
-    const long long o = perm[off + i];
-    const double dx = xyz[3 * o] - c[0], dy = xyz[3 * o + 1] - c[1], dz = xyz[3 * o + 2] - c[2];
+  for (int i = lane; i < cnt; i += 64) {
+    const double dx = s_p[0][i] - s_c[0], dy = s_p[1][i] - s_c[1], dz = s_p[2][i] - s_c[2];
     r = fmax(r, sqrt(dx * dx + dy * dy + dz * dz));
   }
-  for (int k = 0; k < 3; ++k) center[3 * li + k] = c[k];
-  radius[li] = r;
+  for (int w = 32; w > 0; w >>= 1) r = fmax(r, __shfl_xor(r, w, 64));
+  if (lane < 3) center[3 * li + lane] = s_c[lane];
+  if (lane == 0) radius[li] = r;
 }
 
 __device__ __forceinline__ bool significant(const ShellDev &sh, double ext, const double *c,
@@ -256,7 +273,7 @@ void launch_hierarchy(const double *xyz, long long n, int nleaves, double *part,
   if (hipcub::DeviceRadixSort::SortPairs(temp, tb, keys_in, keys_out, idx_in, perm, (int)n, 0, 63,
                                          s) != hipSuccess)
     throw std::runtime_error("hierarchy: radix sort failed");
-  k_leaf_geom<<<(nleaves + 255) / 256, 256, 0, s>>>(xyz, perm, n, nleaves, center, radius);
+  k_leaf_geom<<<nleaves, 64, 0, s>>>(xyz, perm, n, nleaves, center, radius);
   check("hierarchy: leaf spheres");
 }
 
