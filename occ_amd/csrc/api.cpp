@@ -1074,9 +1074,11 @@ void run_gradient(occxc_context *c, const double *d_D, double *d_grad, hipStream
   t.run(OCCXC_STAGE_DENSITY, [&] {
     if (c->mgga)
       mgga_density(c, s);
-    else if (c->plan.use_mfma)
-      run_density(c->plan, a, c->d_ao.get(), c->opt.precision, s);
-    else
+    else if (c->plan.use_mfma) {
+      BuildArgs x = a;
+      x.ao_a = nullptr;  // the gradient needs no A plane
+      run_density(c->plan, x, c->d_ao.get(), c->opt.precision, s);
+    } else
       launch_density_functional(a, c->d_ao.get(), c->opt.precision != OCCXC_PREC_FP64, s);
   });
   t.run(OCCXC_STAGE_GRADIENT, [&] {

@@ -2024,14 +2024,11 @@ __global__ __launch_bounds__(256, 2) void k_den_tile(BuildArgs a, const S *__res
   }
 }
 
-// Leaves with more than one density item: their partials summed in
-// (point block, column block) order, then the functional epilogue.
-__global__ __launch_bounds__(256) void k_den_finish(BuildArgs a, const DenFinish *__restrict__ fin,
-                                                     const double *__restrict__ part) {
-  __shared__ double s_q[4][kMaxLeafPts];
-  __shared__ double s_red[4];
-  const DenFinish F = fin[blockIdx.x];
-  const LeafDev L = a.leaves[F.leaf];
+// A leaf with more than one density item: its partials summed in (point block,
+// column block) order, then the functional epilogue.
+__device__ __forceinline__ void den_finish_leaf(const BuildArgs &a, const DenFinish &F,
+                                                const LeafDev &L, const double *__restrict__ part,
+                                                double (*s_q)[kMaxLeafPts], double *s_red) {
   const int nq = a.deriv ? 4 : 1;
   for (int u = threadIdx.x; u < 4 * L.np; u += blockDim.x) {
     const int k = u / L.np, p = u - k * L.np;
@@ -2045,6 +2042,81 @@ __global__ __launch_bounds__(256) void k_den_finish(BuildArgs a, const DenFinish
   }
   __syncthreads();
   density_epilogue(a, L, F.leaf, s_q, s_red);
+}
+
+__global__ __launch_bounds__(256) void k_den_finish(BuildArgs a, const DenFinish *__restrict__ fin,
+                                                     const double *__restrict__ part) {
+  __shared__ double s_q[4][kMaxLeafPts];
+  __shared__ double s_red[4];
+  const DenFinish F = fin[blockIdx.x];
+  den_finish_leaf(a, F, a.leaves[F.leaf], part, s_q, s_red);
+}
+
+// FP32 mode, what the Vxc stage contracts Phi with: A = sum_q c_q Phi_q of an
+// active leaf (the arithmetic of k_vxc_tile_f32's staging: FP64 sums of the FP32
+// values, rounded to FP32) into a.ao_a at the leaf's res_off, for the leaf's
+// m AOs and np points.  Rows m..mp-1 are left as they are: the contraction
+// reads them, but each of its outputs pairs one row of Phi with one row of
+// A, and the outputs of rows past m are never added into K.  One workgroup per
+// leaf; np / 4 lanes per AO row (4 points each), so a lane's coefficients are
+// fixed.  HBM-bound: 16 bytes read and 4 written per element (GGA), both
+// streamed past the caches (non-temporal: 0.4 ms of 6 on (H2O)128 / def2-SVP).
+template <bool GGA>
+__device__ __forceinline__ void form_a_plane(const BuildArgs &a, const LeafDev &L,
+                                             const float *__restrict__ ao) {
+  const int tpr = L.np >> 2, rpp = 256 / tpr;  // lanes per row, rows per pass
+  const int t = threadIdx.x, row0 = t / tpr;
+  if (row0 >= rpp) return;
+  const int p = 4 * (t - row0 * tpr);
+  constexpr int NQ = GGA ? 4 : 1;
+  double c[NQ][4];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[q][e] = a.coef[q * a.ptot + L.pt_off + p + e];
+  const float *phi = ao + L.ao_off;
+  const long long cs = (long long)L.mp * L.np;
+  float *out = a.ao_a + L.res_off;
+#pragma unroll 2
+  for (int mu = row0; mu < L.m; mu += rpp) {
+    const long long o = (long long)mu * L.np + p;
+    const f4 f = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + o));
+    f4 fx, fy, fz;
+    if constexpr (GGA) {
+      fx = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + cs + o));
+      fy = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + 2 * cs + o));
+      fz = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + 3 * cs + o));
+    }
+    f4 A;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      double v = c[0][e] * (double)f[e];
+      if constexpr (GGA)
+        v += c[1][e] * (double)fx[e] + c[2][e] * (double)fy[e] + c[3][e] * (double)fz[e];
+      A[e] = (float)v;
+    }
+    __builtin_nontemporal_store(A, reinterpret_cast<f4 *>(out + o));
+  }
+}
+
+// FP32 mode: the finish of every leaf (part0 < 0: the leaf's only item has run
+// the functional) and its A plane.  In one kernel the partial sums' and the
+// functional's latencies (0.67 ms of their own on (H2O)128 / def2-SVP, 0.31 ms
+// on a batch of 24 small molecules) pass under other leaves' streaming.
+template <bool GGA>
+__global__ __launch_bounds__(256) void k_den_finish_a(BuildArgs a,
+                                                       const DenFinish *__restrict__ fin,
+                                                       const double *__restrict__ part,
+                                                       const float *__restrict__ ao) {
+  __shared__ double s_q[4][kMaxLeafPts];
+  __shared__ double s_red[4];
+  const DenFinish F = fin[blockIdx.x];
+  const LeafDev L = a.leaves[F.leaf];
+  if (F.part0 >= 0) {
+    den_finish_leaf(a, F, L, part, s_q, s_red);
+    __syncthreads();  // the coefficients and the leaf's flag are written
+  }
+  if (a.leaf_active[F.leaf]) form_a_plane<GGA>(a, L, ao);
 }
 
 // The same sums (nq quantities) to a.rho_out, without the functional.
@@ -2375,57 +2447,8 @@ __global__ __launch_bounds__(256, 2) void k_vxc_tile_f32(BuildArgs a, const floa
   vxc_scatter<true, false>(acc, it, L, MD, map, Km, kScatterCut, reinterpret_cast<double *>(s_stage));
 }
 
-// FP32 mode, first step of the Vxc stage: A = sum_q c_q Phi_q of every active
-// leaf (the arithmetic of k_vxc_tile_f32's staging: FP64 sums of the FP32
-// values, rounded to FP32) into a.ao_a at the leaf's res_off, for the leaf's
-// m AOs and np points.  Rows m..mp-1 are left as they are: the contraction
-// reads them, but each of its outputs pairs one row of Phi with one row of
-// A, and the outputs of rows past m are never added into K.  One workgroup per leaf; np / 4 lanes per AO row (4 points
-// each), so a lane's coefficients are fixed.  HBM-bound: 16 bytes read and 4
-// written per element (GGA), both streamed past the caches (non-temporal:
-// 0.4 ms of 6 on (H2O)128 / def2-SVP).
-template <bool GGA>
-__global__ __launch_bounds__(256) void k_vxc_apass(BuildArgs a, const float *__restrict__ ao) {
-  const int li = blockIdx.x;
-  if (!a.leaf_active[li]) return;
-  const LeafDev L = a.leaves[li];
-  const int tpr = L.np >> 2, rpp = 256 / tpr;  // lanes per row, rows per pass
-  const int t = threadIdx.x, row0 = t / tpr;
-  if (row0 >= rpp) return;
-  const int p = 4 * (t - row0 * tpr);
-  constexpr int NQ = GGA ? 4 : 1;
-  double c[NQ][4];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c[q][e] = a.coef[q * a.ptot + L.pt_off + p + e];
-  const float *phi = ao + L.ao_off;
-  const long long cs = (long long)L.mp * L.np;
-  float *out = a.ao_a + L.res_off;
-#pragma unroll 2
-  for (int mu = row0; mu < L.m; mu += rpp) {
-    const long long o = (long long)mu * L.np + p;
-    const f4 f = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + o));
-    f4 fx, fy, fz;
-    if constexpr (GGA) {
-      fx = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + cs + o));
-      fy = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + 2 * cs + o));
-      fz = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(phi + 3 * cs + o));
-    }
-    f4 A;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      double v = c[0][e] * (double)f[e];
-      if constexpr (GGA)
-        v += c[1][e] * (double)fx[e] + c[2][e] * (double)fy[e] + c[3][e] * (double)fz[e];
-      A[e] = (float)v;
-    }
-    __builtin_nontemporal_store(A, reinterpret_cast<f4 *>(out + o));
-  }
-}
-
 // FP32 mode, second step: the Vxc item's block pair from the Phi and A planes
-// (k_vxc_apass), staged into LDS by direct loads (global_load_lds, 16 bytes
+// (form_a_plane), staged into LDS by direct loads (global_load_lds, 16 bytes
 // a lane) in chunks of kVgP points, two chunk buffers, so the next chunk
 // loads while the MFMAs run on this one and no registers hold staged values.  A
 // buffer holds four operand blocks [Phi rows | A rows | Phi columns | A
@@ -2959,7 +2982,7 @@ double tile_plan_bytes(const LeafDev &L) {
   const double npb = (double)((L.np + kTileAo - 1) / kTileAo);
   const double parts = ncb * npb > 1.0 ? ncb * npb : 0.0;
   return parts * 4 * kTileAo * sizeof(double) + ncb * npb * sizeof(DenItem) +
-         ncb * (ncb + 1) / 2 * sizeof(VxcItem) + sizeof(DenFinish);
+         ncb * (ncb + 1) / 2 * sizeof(VxcItem) + 2 * sizeof(DenFinish);
 }
 
 // Item lists of the tiled path.  The active leaves (Morton order) are cut
@@ -3018,10 +3041,11 @@ std::vector<DenItem> gradient_items(const std::vector<LeafDev> &leaves, int maxw
   return interleave_runs(lists, DenItem{-1, -1, 0, 0, 0, 0});
 }
 
+// form_a: also the list of every leaf for k_den_finish_a (FP32 mode).
 // vxc_only: the Vxc item list alone (FP32 storage without the tiled build
 // kernels needs it once, for dS).
 static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
-                           bool vxc_only = false) {
+                           bool vxc_only = false, bool form_a = false) {
   constexpr int kXcd = kXcdRuns;
   const int nl = (int)leaves.size();
   p.narrow = true;
@@ -3031,7 +3055,7 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
   for (const auto &L : leaves) total += (double)L.np * L.mp * L.mp;
   std::vector<std::vector<DenItem>> den(kXcd);
   std::vector<std::vector<VxcItem>> vxc(kXcd);
-  std::vector<DenFinish> fin;
+  std::vector<DenFinish> fin, all;
   int nparts = 0;
   double acc = 0.0;
   for (int li = 0; li < nl; ++li) {
@@ -3045,6 +3069,7 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
     const auto db = tile_blocks(L.mp, den_ao);
     const bool single = db.size() == 1 && pb.size() == 1;
     if (!single) fin.push_back(DenFinish{li, nparts, (int)db.size(), (int)pb.size()});
+    if (form_a) all.push_back(single ? DenFinish{li, -1, 1, 1} : fin.back());
     for (size_t ip = 0; ip < pb.size(); ++ip)
       for (size_t ic = 0; ic < db.size(); ++ic)
         den[x].push_back(DenItem{li, single ? -1 : nparts + (int)(ip * db.size() + ic),
@@ -3069,10 +3094,15 @@ static void make_tile_plan(ContractPlan &p, const std::vector<LeafDev> &leaves,
     p.den_items.upload(d.data(), d.size());
     p.den_finish.alloc(std::max<size_t>(fin.size(), 1));
     p.den_finish.upload(fin.data(), fin.size());
+    if (form_a) {
+      p.den_finish_all.alloc(std::max<size_t>(all.size(), 1));
+      p.den_finish_all.upload(all.data(), all.size());
+    }
     p.den_part.alloc((size_t)std::max(nparts, 1) * 4 * kTileAo);
   }
   OCCXC_HIP(hipStreamSynchronize(nullptr));  // the host lists are freed on return
-  p.bytes += p.den_items.bytes() + p.vxc_items.bytes() + p.den_finish.bytes() + p.den_part.bytes();
+  p.bytes += p.den_items.bytes() + p.vxc_items.bytes() + p.den_finish.bytes() +
+             p.den_finish_all.bytes() + p.den_part.bytes();
 }
 
 int vxc_variant_setting() {
@@ -3121,7 +3151,7 @@ ContractPlan make_contract_plan(const std::vector<LeafDev> &leaves, long long mt
     p.den_persistent = (p.tune.persistent & 1) != 0;
     const char *dd = std::getenv("OCCXC_DENSITY_DMA");
     p.den_dma = dd ? std::atoi(dd) != 0 : kDefaultDensityDma;
-    make_tile_plan(p, leaves);
+    make_tile_plan(p, leaves, false, precision == 1);
     int dev = 0, cus = 0;
     OCCXC_HIP(hipGetDevice(&dev));
     OCCXC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -3266,7 +3296,12 @@ void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, i
             <<<plan.n_den_items, 256, 0, s>>>(a, x, plan.den_items.get(), plan.den_part.get(),
                                               plan.n_den_items);
       check_launch("k_den_tile");
-      if (plan.n_den_finish > 0) {
+      if (precision == 1 && a.ao_a != nullptr) {
+        (a.deriv ? k_den_finish_a<true> : k_den_finish_a<false>)
+            <<<a.nleaves, 256, 0, s>>>(a, plan.den_finish_all.get(), plan.den_part.get(),
+                                       static_cast<const float *>(ao));
+        check_launch("k_den_finish_a");
+      } else if (plan.n_den_finish > 0) {
         k_den_finish<<<plan.n_den_finish, 256, 0, s>>>(a, plan.den_finish.get(),
                                                        plan.den_part.get());
         check_launch("k_den_finish");
@@ -3392,10 +3427,7 @@ void run_vxc(const ContractPlan &plan, const BuildArgs &a, const void *ao, int p
   if (a.nleaves == 0) return;
   if (plan.tiled) {
     if (precision == 1 && a.ao_a != nullptr) {
-      // FP32 mode with the A plane: A pass, then the directly loaded contraction
-      (a.deriv ? k_vxc_apass<true> : k_vxc_apass<false>)
-          <<<a.nleaves, 256, 0, s>>>(a, static_cast<const float *>(ao));
-      check_launch("k_vxc_apass");
+      // FP32 mode with the A plane, which the density stage has formed
       k_vxc_gemm_f32<<<plan.n_vxc_items, 256, 0, s>>>(a, static_cast<const float *>(ao), a.ao_map,
                                                       plan.vxc_items.get());
       check_launch("k_vxc_gemm_f32");

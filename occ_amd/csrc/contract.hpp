@@ -47,6 +47,7 @@ struct ContractPlan {
   DevBuf<DenItem> den_items;
   DevBuf<VxcItem> vxc_items;
   DevBuf<DenFinish> den_finish;
+  DevBuf<DenFinish> den_finish_all;  // FP32 mode: every leaf (part0 = -1: nothing to finish)
   DevBuf<double> den_part;  // [n_den_parts][4][kTileAo]
   DevBuf<float> d2f;       // FP32 rounding of the doubled density (FP32 mode)
   DevBuf<uint16_t> d2l;    // BF16 rounding of the remainder (FP32 mode)
@@ -68,15 +69,16 @@ int vxc_variant_setting();
 // plan's tiled flag, from the same settings).
 bool tiled_setting(int precision);
 
-// FP32 mode (precision 1), tiled, not meta-GGA: the Vxc stage first forms
-// A = sum_q c_q Phi_q (FP32) of every active leaf in a plane of its own
-// (4 mp np bytes per leaf, held by the context), then contracts Phi with A
-// from LDS filled by direct loads.  OCCXC_VXC_APASS=0 keeps the one-kernel
+// FP32 mode (precision 1), tiled, not meta-GGA: the density stage ends by
+// forming A = sum_q c_q Phi_q (FP32) of every active leaf in a plane of its own
+// (4 mp np bytes per leaf, held by the context), and the Vxc stage contracts Phi
+// with A from LDS filled by direct loads.  OCCXC_VXC_APASS=0 keeps the one-kernel
 // form, which forms A per block pair.
 bool vxc_apass_setting(int precision, bool mgga);
 
 ContractPlan make_contract_plan(const std::vector<LeafDev> &leaves, long long mtot, int deriv,
                                 int precision, hipStream_t s, const TuneChoice &tune = {});
+// with a.ao_a (FP32 mode) it also forms the A plane, which run_vxc then reads
 void run_density(const ContractPlan &plan, const BuildArgs &a, const void *ao, int precision,
                  hipStream_t s);
 // rho and grad rho of every leaf point for the density D2t into a.rho_out
