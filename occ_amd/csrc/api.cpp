@@ -664,7 +664,7 @@ void context_setup(occxc_context *c, int nmol, const occxc_basis *bases,
   c->d_D2.alloc(nn);
   c->k_rep = k_copies(c->mtot);
   c->d_K.alloc(nn * c->k_rep);
-  c->d_V.alloc(nn);
+  c->d_V.alloc(nn + 2 * (size_t)nmol);  // and the packed host path's result
   c->d_coef.alloc((size_t)4 * std::max<long long>(c->ptot, 1));
   c->d_part.alloc((size_t)2 * std::max(c->nleaves, 1));
   c->d_active.alloc((size_t)std::max(c->nleaves, 1));
@@ -770,7 +770,7 @@ void context_setup(occxc_context *c, int nmol, const occxc_basis *bases,
     a.ntchunks = (int)tchunks.size();
     a.tpartial = c->d_tpartial.get();
   }
-  c->device_bytes = ao_bytes + ds_bytes + c->d_D.bytes() * 3 + c->d_K.bytes() + c->d_coef.bytes() + c->d_px.bytes() * 4 +
+  c->device_bytes = ao_bytes + ds_bytes + c->d_D.bytes() * 2 + c->d_V.bytes() + c->d_K.bytes() + c->d_coef.bytes() + c->d_px.bytes() * 4 +
                     c->d_porig.bytes() +
                     c->d_ao_map.bytes() + c->d_leaves.bytes() + c->d_leaf_shells.bytes() +
                     c->plan.bytes + c->d_kloc.bytes() + c->d_tpairs.bytes() +
@@ -1430,6 +1430,11 @@ occxc_status occxc_build_device(occxc_context *ctx, const double *d_D, double *d
   });
 }
 
+// Matrix elements up to which the host builds copy through one packed buffer:
+// a copy call costs about 10 us whatever its size, the buffer's extra pass over
+// host memory as much at half a megabyte.
+constexpr size_t kPackedElems = 65536;
+
 occxc_status occxc_batch_build(occxc_context *ctx, const double *const *D, double *const *Vxc,
                                double *exc, double *nelec) {
   return guarded([&] {
@@ -1440,6 +1445,24 @@ occxc_status occxc_batch_build(occxc_context *ctx, const double *const *D, doubl
       const size_t nn = (size_t)ctx->mol_nbf[m] * ctx->mol_nbf[m];
       for (size_t i = 0; i < nn; ++i)
         OCCXC_REQUIRE(std::isfinite(D[m][i]), OCCXC_ERR_INVALID_ARGUMENT, "D: non-finite entry");
+    }
+    const size_t mtot = (size_t)ctx->mtot, nres = 2 * (size_t)ctx->nmol;
+    if (mtot <= kPackedElems) {
+      // small matrices: one copy each way instead of one per molecule and the
+      // scalars, through a packed host buffer (the result behind Vxc)
+      std::vector<double> host(mtot + nres);
+      for (int m = 0; m < ctx->nmol; ++m)
+        std::copy_n(D[m], (size_t)ctx->mol_nbf[m] * ctx->mol_nbf[m], host.data() + ctx->mol_off[m]);
+      ctx->d_D.upload(host.data(), mtot, ctx->stream);
+      launch_build(ctx, ctx->d_D.get(), ctx->d_V.get(), ctx->d_V.get() + mtot, ctx->stream);
+      ctx->d_V.download(host.data(), mtot + nres, ctx->stream);
+      OCCXC_HIP(hipStreamSynchronize(ctx->stream));
+      for (int m = 0; m < ctx->nmol; ++m) {
+        std::copy_n(host.data() + ctx->mol_off[m], (size_t)ctx->mol_nbf[m] * ctx->mol_nbf[m], Vxc[m]);
+        exc[m] = host[mtot + 2 * m];
+        nelec[m] = host[mtot + 2 * m + 1];
+      }
+      return;
     }
     for (int m = 0; m < ctx->nmol; ++m) {
       const size_t nn = (size_t)ctx->mol_nbf[m] * ctx->mol_nbf[m];
