@@ -14,43 +14,25 @@
 // Layout: the context's points are in leaf order; k_vv10_prep scatters each
 // real point's (x, y, z, rho w, omega0, kappa, rho) into input-order planes
 // of npts; k_vv10_pairs gives partial sums of F, U, W per input point and
-// segment of j; k_vv10_coef adds them up per leaf point and forms the weighted
+// segment of j (nlc_segments.hpp); k_vv10_coef adds them up per leaf point and forms the weighted
 // exc / vrho / vsigma and the GGA Vxc coefficients, which the restricted Vxc
 // kernel contracts (Vxc = ktmp + ktmp^T, nonlocal_correlation.cpp:295-303).
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cmath>
 #include <stdexcept>
 #include <string>
 
 #include "kernels.hpp"
+#include "nlc_segments.hpp"
 
 namespace occxc {
 namespace {
 
 constexpr double kVvPi = 3.14159265358979323846;
 constexpr double kVvRhoMin = 1e-8;  // nonlocal_correlation.cpp:68,77
-constexpr int kVvTile = 256;   // j points of a tile
-constexpr int kVvRows = 512;   // i points of a block, two per thread
-constexpr int kVvSegs = 16;    // most segments of j
 
 enum : int { kX = 0, kY, kZ, kRW, kOM, kKA, kRHO, kNlcPlanes };
-
-// Segments of j: runs of `tiles` tiles, so that the triangle of pairs becomes
-// many units of about equal work (one workgroup per 256 points with all of its
-// j tiles left a quarter of the chip idle at the end: 1032 workgroups, all
-// resident at once, the longest twice the average).
-struct VvSegs {
-  int tiles, n;
-};
-VvSegs vv_segs(long long npts) {
-  const long long nt = (npts + kVvTile - 1) / kVvTile;
-  VvSegs g;
-  g.tiles = (int)std::max<long long>(8, (nt + kVvSegs - 1) / kVvSegs);
-  g.n = (int)std::max<long long>(1, (nt + g.tiles - 1) / g.tiles);
-  return g;
-}
 
 void check(const char *what) {
   const hipError_t e = hipGetLastError();
@@ -189,9 +171,9 @@ __global__ __launch_bounds__(256) void k_vv10_pairs(const double *__restrict__ n
   __shared__ double2 s_xy[kVvTile], s_zq[kVvTile], s_ok[kVvTile];
   const long long b = (long long)gridDim.x - 1 - blockIdx.x;
   const int seg = blockIdx.y;
+  if (seg >= vv_block_segs(b, npts, seg_tiles)) return;
   const long long jt0 = (long long)seg * seg_tiles;
-  if (jt0 > 2 * b + 1) return;
-  const long long jt1 = min(jt0 + seg_tiles, 2 * b + 2);
+  const long long jt1 = min(jt0 + seg_tiles, vv_last_tile(b, npts) + 1);
   VvPoint p[2];
   long long i[2];
   bool live[2], wide = false;
@@ -301,7 +283,7 @@ __global__ __launch_bounds__(256) void k_vv10_coef(BuildArgs a, const double *__
       const double dka_dr = (1.0 / 6.0) * ka;
       // the segments that the point's block has, in order
       double F = 0.0, U = 0.0, W = 0.0;
-      const int nseg = (int)((2 * (o / kVvRows) + 1) / seg_tiles) + 1;
+      const int nseg = vv_block_segs(o / kVvRows, npts, seg_tiles);
       for (int g = 0; g < nseg; ++g) {
         const double *f = part + 3 * (long long)g * npts + o;
         F += f[0];
@@ -344,8 +326,7 @@ void launch_vv10(const BuildArgs &a, const double *rho4, const int *porig, doubl
   launch_zero(nlc + kRHO * npts, npts, s);
   k_vv10_prep<<<a.nleaves, 256, 0, s>>>(a, rho4, porig, k, nlc, npts);
   check("k_vv10_prep");
-  const long long nblk = (npts + kVvRows - 1) / kVvRows;
-  k_vv10_pairs<<<dim3((unsigned)nblk, g.n), 256, 0, s>>>(nlc, npts, g.tiles, part);
+  k_vv10_pairs<<<dim3((unsigned)vv_blocks(npts), g.n), 256, 0, s>>>(nlc, npts, g.tiles, part);
   check("k_vv10_pairs");
   k_vv10_coef<<<a.nleaves, 256, 0, s>>>(a, rho4, porig, k, part, npts, g.tiles);
   check("k_vv10_coef");

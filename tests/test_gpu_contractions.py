@@ -120,3 +120,24 @@ def test_vv10_matches_oracle(shift, b, nrad, nang):
     ctx.close()
     assert abs(got - e) <= 1e-12 * abs(e)
     assert np.abs(K - V).max() <= 1e-11 + 1e-11 * np.abs(V).max()
+
+
+# More than 32,768 points, where segments of j are longer than eight tiles: 135
+# tiles (15 segments of 9, the last block's second tile missing) and 136, the
+# last input points next to the nuclei.  Bounds as above.
+@pytest.mark.parametrize("npts", [34305, 34400, 34816])
+def test_vv10_segments_with_live_last_points(npts):
+    atoms = molecules.water()
+    basis = AOBasis.load(atoms, "6-31g")
+    pts, wts = MolecularGrid(atoms, GridSettings(radial_points=75, angular_points=302)).build()
+    d = np.min([np.linalg.norm(pts - np.array(a[1:]), axis=1) for a in atoms], axis=0)
+    near = np.argsort(-d, kind="stable")[-npts:]  # the nearest npts points, far to near
+    pts, wts = np.ascontiguousarray(pts[near]), np.ascontiguousarray(wts[near])
+    print(f"vv10 npts={len(wts)}", flush=True)
+    D = random_density(basis.nbf, 5, 43)
+    e, V = oracle.vv10(oracle.OracleBasis.from_flat(basis.flat()), pts, wts, D, b=6.0, C=0.01)
+    ctx = XCContext(basis, pts, wts, functional_ids("pbe"))
+    got, K = ctx.nlc_vv10(D, b=6.0, C=0.01)
+    ctx.close()
+    assert abs(got - e) <= 1e-12 * abs(e)
+    assert np.abs(K - V).max() <= 1e-11 + 1e-11 * np.abs(V).max()
