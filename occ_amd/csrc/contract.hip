@@ -30,6 +30,7 @@
 
 #include "contract.hpp"
 #include "tile_dma.hpp"
+#include "tile_shapes.hpp"
 #include "tuning_table.hpp"
 #include "xc_functionals.hpp"
 
@@ -2960,21 +2961,6 @@ void check_coef_planes(int need, int have, const char *what) {
 static size_t vxc_smem(size_t elem) {
   const size_t pad = 16 / elem;
   return sizeof(double) * 4 * kMaxLeafPts + elem * 64 * (128 + pad);
-}
-
-// Blocks of a leaf's padded AOs: n / 32 units of 32 split into the fewest
-// blocks of at most maxw / 32 units, the first ones one unit larger.
-static std::vector<std::pair<int, int>> tile_blocks(int n, int maxw = kTileAo) {
-  std::vector<std::pair<int, int>> b;
-  const int per = std::max(1, maxw / 32);
-  const int units = n / 32, nb = (units + per - 1) / per;
-  int at = 0;
-  for (int k = 0; k < nb; ++k) {
-    const int u = units / nb + (k < units % nb ? 1 : 0);
-    b.push_back({at, 32 * u});
-    at += 32 * u;
-  }
-  return b;
 }
 
 double tile_plan_bytes(const LeafDev &L) {

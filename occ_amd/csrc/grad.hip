@@ -31,6 +31,7 @@
 
 #include "kernels.hpp"
 #include "tile_dma.hpp"
+#include "tile_shapes.hpp"
 
 namespace occxc {
 
@@ -150,7 +151,9 @@ __device__ __forceinline__ void grad_item(const BuildArgs &a, const S *__restric
   };
   double(*s_c)[kGp] = reinterpret_cast<double(*)[kGp]>(s_stage + P::NS * P::STAGE);
   const int nch = (L.m + kGk - 1) / kGk;
-  const int CTl = live_tiles(L.m - (it.c0 + wc * hc), hc);
+  // exactly the tiles that hold real AOs: the integrand reads its columns' rows
+  // from memory, and in a block of 32 a half has one tile
+  const int CTl = half_tiles(L.m - (it.c0 + wc * hc), hc);
   double gs[CT][3];
 #pragma unroll
   for (int j = 0; j < CT; ++j) gs[j][0] = gs[j][1] = gs[j][2] = 0.0;
@@ -278,6 +281,7 @@ __device__ __forceinline__ void grad_item(const BuildArgs &a, const S *__restric
   };
   switch (CTl) {
   case 0: body(std::integral_constant<int, 0>{}); break;
+  case 1: body(std::integral_constant<int, 1>{}); break;
   case 2: body(std::integral_constant<int, 2>{}); break;
   case 3: body(std::integral_constant<int, CT < 3 ? CT : 3>{}); break;
   default: body(std::integral_constant<int, CT>{}); break;

@@ -4,15 +4,16 @@
 
 #include <hip/hip_runtime.h>
 
+#include "tile_shapes.hpp"
+
 namespace occxc {
 namespace {
 
-// 16-row tiles of a wavefront's half block (half rows) that hold any of the
-// `valid` rows counted from its first row: the tiles past a leaf's real AOs
-// or points hold padding only (zero AO rows, zero-weight points) and are not
-// computed.  One tile runs as the 2-tile shape (the shapes start at 2).
+// Tiles that the contractions run for a wavefront's half block (half_tiles); one
+// tile runs as the 2-tile shape (their shapes start at 2, and the second tile's
+// operands are in LDS whatever the width of the block).
 __device__ __forceinline__ int live_tiles(int valid, int half) {
-  const int t = (min(max(valid, 0), half) + 15) >> 4;
+  const int t = half_tiles(valid, half);
   return t == 1 ? 2 : t;
 }
 

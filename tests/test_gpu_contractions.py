@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 SYSTEMS = {"water": lambda: molecules.water(), "methane": lambda: molecules.alkane(1),
            "water3": lambda: molecules.water_cluster(3, seed=6),
-           "alkane5": lambda: molecules.alkane(5)}
+           "alkane3": lambda: molecules.alkane(3), "alkane5": lambda: molecules.alkane(5)}
 
 
 def _setup(system, basis_name, method, precision, tile, nrad=19, nang=38):
@@ -98,6 +98,16 @@ def test_gradients_match_oracle(system, basis_name, method, precision):
     got = ctx.xc_gradient_unrestricted(Du, basis.shell_atom, n)
     assert np.abs(got - Gu).max() <= tol * max(1.0, np.abs(Gu).max())
     ctx.close()
+
+
+# the same with column blocks of 32 AOs whose second half holds real ones: one
+# block of 17 to 32 AOs, and for a meta-GGA 64 + 32 with more than 80
+@pytest.mark.parametrize("precision", ["fp64", "fp32cache"])
+@pytest.mark.parametrize("method", ["svwn5", "pbe", "tpss"])
+@pytest.mark.parametrize("system,basis_name", [
+    ("methane", "6-31g"), ("water", "def2-svp"), ("alkane3", "def2-svp")])
+def test_gradients_of_blocks_of_32(system, basis_name, method, precision):
+    test_gradients_match_oracle(system, basis_name, method, precision)
 
 
 # VV10: one pass over several segments of j, points within and beyond the range
