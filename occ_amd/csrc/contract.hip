@@ -2153,7 +2153,9 @@ __global__ __launch_bounds__(256) void k_den_finish_store(BuildArgs a,
 // 3.6 on (H2O)32); in the register-staged ones the atomics drain behind other
 // workgroups' staging and the fold's barriers cost more than it saves.
 // MT: tiles of a wavefront each way (4, or 2 for blocks of at most 64 AOs).
-template <bool F32, bool FOLD, int MT = 4>
+// CUT = false: every entry is added, NaN included (zeros, which change nothing,
+// are left out).
+template <bool F32, bool FOLD, int MT = 4, bool CUT = true>
 __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[MT][MT], const VxcItem &it,
                                             const LeafDev &L, const MolDev &MD,
                                             const int *__restrict__ map, double *Km, double cut,
@@ -2177,7 +2179,7 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[MT][MT], const VxcIt
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int mu = it.r0 + wr * hr + lrow(i, r);
-          if (mu < L.m && fabs(acc[i][j][r]) >= cut)
+          if (mu < L.m && (CUT ? fabs(acc[i][j][r]) >= cut : acc[i][j][r] != 0.0))
             atomicAdd(kc + (long long)map[mu] * MD.nbf, acc[i][j][r]);
         }
       }
@@ -2203,10 +2205,10 @@ __device__ __forceinline__ void vxc_scatter(const d4 (&acc)[MT][MT], const VxcIt
   // FP64: the two terms of a folded entry are screened one by one, as the
   // unfolded scatter screens them, so the fold drops nothing more
   auto kept = [&](double v) __attribute__((always_inline)) {
-    return F32 || fabs(v) >= cut ? v : 0.0;
+    return F32 || !CUT || fabs(v) >= cut ? v : 0.0;
   };
   auto emit = [&](int i, int j, int r, double v) __attribute__((always_inline)) {
-    if (ro[i][r] >= 0 && co[j] >= 0 && (F32 ? fabs(v) >= cut : v != 0.0))
+    if (ro[i][r] >= 0 && co[j] >= 0 && (F32 && CUT ? fabs(v) >= cut : v != 0.0))
       atomicAdd(Km + ro[i][r] + co[j], v);
   };
   // [row][col ^ (row % 16)] keeps a wavefront's column reads off one bank
@@ -2755,7 +2757,9 @@ __device__ __forceinline__ void vxc_item_dma(const BuildArgs &a, const S *__rest
       }
     }
   });
-  vxc_scatter<false, true, MT>(acc, it, L, MD, map, Km, TAU ? kStorageCut : kScatterCut, reinterpret_cast<double *>(s_stage));
+  // a meta-GGA's entries are all added, as the per-leaf kernels add them
+  vxc_scatter<false, true, MT, !TAU>(acc, it, L, MD, map, Km, kScatterCut,
+                                     reinterpret_cast<double *>(s_stage));
 }
 
 template <typename S, bool GGA, bool TAU, int MT>

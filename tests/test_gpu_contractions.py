@@ -151,3 +151,24 @@ def test_vv10_segments_with_live_last_points(npts):
     ctx.close()
     assert abs(got - e) <= 1e-12 * abs(e)
     assert np.abs(K - V).max() <= 1e-11 + 1e-11 * np.abs(V).max()
+
+
+# A meta-GGA's potential is added in full: with weights of 1e-16 of a grid's all
+# entries are that small, and none may be left out (1e-11 of the largest, as
+# above).
+@pytest.mark.parametrize("tile", [0, 32, 64])
+@pytest.mark.parametrize("precision", ["fp64", "fp32cache"])
+def test_meta_gga_potential_is_added_in_full(precision, tile):
+    basis, pts, wts, ctx = _setup("water3", "def2-svp", "tpss", precision, tile)
+    ctx.close()
+    wts = 1e-16 * wts
+    ctx = XCContext(basis, pts, wts, functional_ids("tpss"), precision=precision, tile_ao=tile)
+    D = random_density(basis.nbf, 5, 17)
+    ob, ids = oracle.OracleBasis.from_flat(basis.flat()), functional_ids("tpss")
+    tol = 1e-11 if precision == "fp64" else 1e-7
+    K = oracle.xc_build(ob, pts, wts, ids, D)[0]
+    assert np.abs(ctx.build(D)[0] - K).max() <= tol * np.abs(K).max()
+    Du = np.asfortranarray(np.concatenate([D, random_density(basis.nbf, 4, 22)]) / 2)
+    K = oracle.xc_build_unrestricted(ob, pts, wts, ids, Du)[0]
+    assert np.abs(ctx.build_unrestricted(Du)[0] - K).max() <= tol * np.abs(K).max()
+    ctx.close()
