@@ -1258,13 +1258,12 @@ void uks_setup(occxc_context *c) {
   c->uks_ready = true;
 }
 
-// Device copies of D and Vxc (2 nbf x nbf) for the host entry points.
-void uks_host_buffers(occxc_context *c) {
+// The host entry points' device matrix (2 nbf x nbf): D, and then Vxc in its
+// place (a build reads D before it writes Vxc).
+void uks_host_buffer(occxc_context *c) {
   if (c->d_Du.size()) return;
-  const size_t nn = (size_t)c->nbf * c->nbf;
-  c->d_Du.alloc(2 * nn);
-  c->d_Vu.alloc(2 * nn);
-  c->device_bytes += c->d_Du.bytes() + c->d_Vu.bytes();
+  c->d_Du.alloc(2 * (size_t)c->nbf * c->nbf);
+  c->device_bytes += c->d_Du.bytes();
 }
 
 void drop_graph(occxc_context *c) {
@@ -1591,10 +1590,10 @@ occxc_status occxc_build_unrestricted(occxc_context *ctx, const double *D, doubl
       OCCXC_REQUIRE(std::isfinite(D[i]), OCCXC_ERR_INVALID_ARGUMENT, "D: non-finite entry");
     DeviceGuard g(ctx->device);
     uks_setup(ctx);
-    uks_host_buffers(ctx);
+    uks_host_buffer(ctx);
     ctx->d_Du.upload(D, 2 * nn, ctx->stream);
-    run_build_u(ctx, ctx->d_Du.get(), ctx->d_Vu.get(), ctx->d_result_u.get(), ctx->stream);
-    ctx->d_Vu.download(Vxc, 2 * nn, ctx->stream);
+    run_build_u(ctx, ctx->d_Du.get(), ctx->d_Du.get(), ctx->d_result_u.get(), ctx->stream);
+    ctx->d_Du.download(Vxc, 2 * nn, ctx->stream);
     double r[3];
     ctx->d_result_u.download(r, 3, ctx->stream);
     OCCXC_HIP(hipStreamSynchronize(ctx->stream));
@@ -1658,7 +1657,7 @@ occxc_status occxc_xc_gradient_unrestricted(occxc_context *ctx, const double *D,
       OCCXC_REQUIRE(std::isfinite(D[i]), OCCXC_ERR_INVALID_ARGUMENT, "D: non-finite entry");
     DeviceGuard g(ctx->device);
     gradient_u_prepare(ctx, natoms, shell_atom);
-    uks_host_buffers(ctx);
+    uks_host_buffer(ctx);
     ctx->d_Du.upload(D, 2 * nn, ctx->stream);
     run_gradient_u(ctx, ctx->d_Du.get(), ctx->d_grad.get(), ctx->stream);
     ctx->d_grad.download(grad, 3 * (size_t)natoms, ctx->stream);

@@ -81,9 +81,9 @@ struct occxc_context {
   // unrestricted builds (allocated on the first one): 2 D_s^T per spin, rho and
   // grad rho per spin, the beta-spin coefficients and K (alpha uses the
   // restricted buffers; d_V_b in the two-pass form only), per-leaf {Exc,
-  // N_alpha, N_beta} and the result; for the host entry points D and Vxc
-  // (2 nbf x nbf)
-  occxc::DevBuf<double> d_Du, d_Vu, d_D2a, d_D2b, d_rho_a, d_rho_b, d_coef_b, d_K_b, d_V_b, d_part_u,
+  // N_alpha, N_beta} and the result; for the host entry points one 2 nbf x nbf
+  // matrix, which takes D in and Vxc out
+  occxc::DevBuf<double> d_Du, d_D2a, d_D2b, d_rho_a, d_rho_b, d_coef_b, d_K_b, d_V_b, d_part_u,
       d_result_u;
   bool uks_ready = false;
   // restricted meta-GGA (allocated at context creation): rho and grad rho

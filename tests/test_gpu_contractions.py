@@ -172,3 +172,25 @@ def test_meta_gga_potential_is_added_in_full(precision, tile):
     K = oracle.xc_build_unrestricted(ob, pts, wts, ids, Du)[0]
     assert np.abs(ctx.build_unrestricted(Du)[0] - K).max() <= tol * np.abs(K).max()
     ctx.close()
+
+
+# The host entry points keep one 2 nbf x nbf matrix beside what the device ones
+# keep (allocated whole or not at all), D going in and Vxc coming out of it.
+@pytest.mark.parametrize("method", ["pbe", "tpss"])
+def test_unrestricted_host_build_keeps_one_matrix(method):
+    from occ_amd.device import DeviceArray
+    basis, pts, wts, ctx = _setup("water3", "6-31g", method, "fp64", 0)
+    n = basis.nbf
+    D = np.asfortranarray(np.concatenate([random_density(n, 5, 21), random_density(n, 4, 22)]) / 2)
+    dD, dV, dr = DeviceArray(2 * n * n), DeviceArray(2 * n * n), DeviceArray(3)
+    dD.upload(D)
+    ctx.build_unrestricted_device(dD.ptr, dV.ptr, dr.ptr)
+    ctx.synchronize()
+    on_device = ctx.info()["device_bytes"]
+    first, second = ctx.build_unrestricted(D), ctx.build_unrestricted(D)
+    assert ctx.info()["device_bytes"] - on_device == 16 * n * n
+    # FP64 atomics: equal to rounding
+    for V, e, nel in (first, second):
+        assert np.abs(V - dV.download((2 * n, n))).max() <= 1e-13
+        assert [e, *nel] == list(dr.download())
+    ctx.close()
