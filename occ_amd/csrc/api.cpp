@@ -1040,6 +1040,7 @@ void gradient_setup(occxc_context *c, int natoms, const int *shell_atom) {
   const bool same = c->grad_natoms == natoms && (int)c->grad_shell_atom.size() == c->nsh &&
                     std::equal(shell_atom, shell_atom + c->nsh, c->grad_shell_atom.begin());
   if (same) return;
+  c->grad_natoms = 0;  // no map is set up until the lists and buffers below are whole
   std::vector<int> map(c->d_ao_map.size());
   c->d_ao_map.download(map.data(), map.size(), c->stream);
   OCCXC_HIP(hipStreamSynchronize(c->stream));
