@@ -41,7 +41,7 @@ struct occxc_context {
   // dS = sum_p w_p (r Phi^T + Phi r^T), the first-order change of the grid
   // overlap from the stored values to the exact ones
   occxc::DevBuf<float> d_ao_res;
-  occxc::DevBuf<float> d_ao_a;  // FP32 mode: the Vxc stage's A plane (A pass)
+  occxc::DevBuf<float> d_ao_a;  // FP32 mode: the A plane, formed by the density stage
   occxc::DevBuf<double> d_dS, d_ncorr;
   int k_rep = 1;  // copies of K (k_copies)
   occxc::DevBuf<double> d_D, d_D2, d_K, d_V, d_coef, d_part, d_result;
@@ -96,7 +96,8 @@ struct occxc_context {
   // d_mtau / d_coef_tau), and D_s + D_s^T per spin for the tau passes
   occxc::DevBuf<double> d_mtau_b, d_coef_tau_b, d_D2sa, d_D2sb;
   occxc::DevBuf<occxc::LeafDev> d_leaves_k;
-  // VV10 (allocated on the first call): input-order point planes and F, U, W
+  // VV10 (allocated on the first call): seven input-order point planes, then
+  // three planes of partial F, U, W per segment of j (nlc_segments.hpp)
   occxc::DevBuf<double> d_nlc;
 };
 

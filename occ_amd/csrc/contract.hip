@@ -1439,8 +1439,8 @@ __global__ __launch_bounds__(256) void k_vxc_reduce_final(BuildArgs a, double *_
 // wavefront works on a 2D block of up to 4 x 4 16x16 MFMA tiles (FP64
 // arithmetic; S is the AO storage type).
 
-// Vxc scatter screening: a block entry below kScatterCut in magnitude is not
-// added into K.  An entry of Vxc = K + K^T gathers at most two terms per
+// Vxc scatter screening (LDA and GGA): a block entry below kScatterCut in
+// magnitude is not added into K.  An entry of Vxc = K + K^T gathers at most two terms per
 // leaf, so the change of any Vxc entry is below 2 kScatterCut times the
 // number of leaves (under 2e-9 for 1e5 leaves, against the 1e-7 tolerance);
 // Exc and N_elec are not affected.  About half the block entries are that small (AO pairs
@@ -2583,9 +2583,10 @@ __global__ __launch_bounds__(256, 2) void k_vxc_gemm_f32(BuildArgs a, const floa
 // busy 37 %, 3.7 TB/s).  Forming Phi and A in LDS by way of registers (each
 // element's four planes loaded and waited for by the thread that stores it)
 // took 4.12 ms there; the meta-GGA's passes of per-leaf kernels 23.7 ms, this
-// form 6.46 ms (2.9 times the MFMAs; its scatter drops nothing above 1e-18).  A chunk's operands fill the registers (128 of the 256
-// hold accumulators): Phi is read last, and TAU keeps its plane loop rolled,
-// without which 18 and 40 of them spill.
+// form 6.36 ms (2.9 times the MFMAs; its scatter adds every entry, which costs
+// nothing measurable: 14.87 -> 14.85 ms a build).  A chunk's operands fill the
+// registers (128 of the 256 hold accumulators): Phi is read last, and TAU keeps
+// its plane loop rolled, without which 18 and 40 of them spill.
 // MT = 2: a context whose blocks are all at most 64 AOs wide; half the LDS and
 // a quarter of the accumulators, so that four workgroups share a CU.
 constexpr int kVdRow = 64;                                        // bytes of a row in a chunk

@@ -67,11 +67,11 @@ template <typename T> __device__ __forceinline__ const T *at(const T *base, unsi
 // in flight; every wavefront issues the same number of loads for a chunk.
 // Bound by HBM: the nine derivative planes of the integrand are read once
 // (1.9e10 bytes on (H2O)32 / def2-SVP, FP64), the four of the products once per
-// column block: 3.6e10 bytes past L2 in all.  PBE there 11.76 -> 6.70 ms (5.4
+// column block: 3.6e10 bytes past L2 in all.  PBE there 11.76 -> 6.48 ms (5.6
 // TB/s) against the per-leaf form, which read the products' planes once per 32
-// AOs through each lane's own loads (5.7e10 bytes); the
-// TPSS terms of C11H24, 5.95 -> 2.53 ms for both spins (five products of two
-// kernels then, four of one now).
+// AOs through each lane's own loads (5.7e10 bytes); the TPSS terms of C11H24,
+// 5.98 -> 2.40 ms for both spins (five products of two kernels then, four of one
+// now; 2.59 ms while a half with one tile ran two).
 constexpr int kGk = 8, kGp = kGradPoints;
 template <typename S, int NT> struct GradDma {
   static constexpr int NS = 3;

@@ -778,7 +778,6 @@ __global__ void k_functional_mgga_points(int id, long long n, const double *__re
   if (fam == 2) vtau[i] += vt;
 }
 
-// {Exc, N_alpha, N_beta}: fixed-order sums of the per-leaf partials
 // Polarised functionals over points (libxc layout), ADDING to the outputs.
 __global__ void k_functional_pol_points(int id, long long n, const double *__restrict__ rho,
                                         const double *__restrict__ sigma,

@@ -159,7 +159,7 @@ struct BuildArgs {
   float *ao_res;
   int res_leaf0, res_leaf1;
   long long res_base;
-  // FP32 mode with the A pass: A = sum_q c_q Phi_q of every active leaf,
+  // FP32 mode with the A plane: A = sum_q c_q Phi_q of every active leaf,
   // [mp][np] per leaf at res_off (null otherwise)
   float *ao_a;
   double *kloc;         // two-pass Vxc: per-leaf K_loc blocks (null: atomics into K)
@@ -289,7 +289,8 @@ void launch_functional_mgga(int id, long long n, const double *rho, const double
 // VV10 (nlc.hip): from rho / grad rho of the leaf points (rho4, [4][ptot])
 // and each padded point's input index (porig), the weighted VV10 exc / vrho /
 // vsigma as GGA Vxc coefficients in a.coef and {E_nlc, N_elec} per leaf in
-// a.leaf_part (every leaf active); nlc holds nlc_buffer_elems(npts) doubles
+// a.leaf_part (every leaf active); nlc holds nlc_buffer_elems(npts) doubles, 10
+// to 55 a point
 size_t nlc_buffer_elems(long long npts);
 void launch_vv10(const BuildArgs &a, const double *rho4, const int *porig, double b, double C,
                  double *nlc, long long npts, hipStream_t s);

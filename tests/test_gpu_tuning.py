@@ -91,7 +91,7 @@ def test_density_staging_forms_agree(monkeypatch, precision):
 @pytest.mark.parametrize("deriv_ids", ["gga", "lda"])
 def test_fp32_vxc_forms_agree(monkeypatch, deriv_ids):
     """FP32 mode's Vxc stage in its two forms: A = sum_q c_q Phi_q formed once
-    per leaf (k_vxc_apass) and contracted from directly loaded LDS with the
+    per leaf (k_den_finish_a) and contracted from directly loaded LDS with the
     diagonal blocks folded before the scatter (the default), and the
     one-kernel form that forms A per block pair (OCCXC_VXC_APASS=0).  Both
     round A to FP32 the same way and sum 32 points at a time in FP32 but in a
