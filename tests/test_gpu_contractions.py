@@ -4,7 +4,7 @@ to four blocks per leaf, every form (LDA, GGA, meta-GGA; one spin and two)
 and both storage precisions, against the CPU oracle.
 
 Bounds on Vxc in FP64: each leaf drops at most two terms below 1e-14 per
-entry (none above 1e-18 for a meta-GGA) and the sums round at 1e-15 of the
+entry (none for a meta-GGA) and the sums round at 1e-15 of the
 largest entry per leaf, so 2e-14 leaves + 1e-13 max|V|, below 1e-11 here.
 FP32 AO storage rounds each value by 6e-8 relative: 1e-7 max|V|, the bound of
 the batch tests."""
